@@ -316,8 +316,9 @@ int stda_hip_format_curve(int64_t n, const double *e, const double *r, char *out
  *   1 mixed: the transition-density contractions (Q gamma Q^T products) in
  *     FP32 with FP32 accumulation, Davidson orthogonalisation, Rayleigh-Ritz
  *     and residual norms in FP64, converged to a residual of 1e-6, followed
- *     by one FP64 Rayleigh-Ritz refinement of the converged roots.  The
- *     response solver uses the FP32 operator with a 1e-6 tolerance.
+ *     by FP64 refinement of the converged roots (TDA: up to four iterations,
+ *     to 1e-7; RPA: one Rayleigh-Ritz step).  The response solver uses the
+ *     FP32 operator with a 1e-6 tolerance.
  *   2 split-bfloat16: the same, with the operator GEMMs' FP32 operands split
  *     into two bfloat16 numbers each and multiplied as hi*hi + hi*lo + lo*hi
  *     on the bfloat16 matrix cores with FP32 accumulation, to a residual of
@@ -336,6 +337,15 @@ int stda_hip_set_precision(stda_hip_ctx *ctx, int32_t precision);
 int stda_hip_gemm(stda_hip_ctx *ctx, int32_t mode, int32_t ta, int32_t tb, int32_t m, int32_t n,
                   int32_t k, double alpha, const double *A, int64_t lda, const double *B,
                   int64_t ldb, double beta, double *C, int64_t ldc);
+
+/* The k lowest eigenpairs of a symmetric matrix (n x n, column-major; n <= 192,
+ * k <= min(n, 32)) with the kernel of the eigensolver's subspace step: w[k]
+ * ascending, z (n x k) orthonormal.  *ok = 0 when eigenvalues lie too close for
+ * it (then w and z are not to be used; the solvers take the host's LAPACK).
+ * No counterpart in the reference (its ssyevr/ssyevd); exposes the kernel to
+ * tests and to callers that want it. */
+int stda_hip_sym_lowest(stda_hip_ctx *ctx, int32_t n, int32_t k, const double *a, double *w,
+                        double *z, int32_t *ok);
 
 /* Timing of the last setup/solve phases on this context, in milliseconds:
  * [0] gamma+charges+intermediates, [1] screening+sort, [2] PT2,

@@ -42,6 +42,7 @@ C_API = [
     "stda_hip_prepare_ao", "stda_hip_index_size", "stda_hip_gspec_noalloc", "stda_hip_gemm",
     "stda_hip_batch_submit", "stda_hip_batch_result", "stda_hip_batch_stop",
     "stda_hip_batch_configure_wide", "stda_hip_batch_wide_count", "stda_hip_batch_set_precision",
+    "stda_hip_sym_lowest",
 ]
 
 
@@ -109,6 +110,7 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     L.stda_hip_timings.argtypes = [P, P]
     L.stda_hip_set_precision.argtypes = [P, I32]
     L.stda_hip_gemm.argtypes = [P, I32, I32, I32, I32, I32, I32, F64, P, I64, P, I64, F64, P, I64]
+    L.stda_hip_sym_lowest.argtypes = [P, I32, I32, P, P, P, ctypes.POINTER(I32)]
     L.stda_hip_load.argtypes = [P, ctypes.POINTER(_System), ctypes.POINTER(_Params)]
     L.stda_hip_select.argtypes = [P, ctypes.POINTER(I64), ctypes.POINTER(I64), ctypes.POINTER(I64)]
     L.stda_hip_kernel_stats.argtypes = [P, ctypes.c_char_p, ctypes.POINTER(F64),
@@ -275,6 +277,16 @@ class StdaHip:
                                           max(1, A.shape[0]), _ptr(B), max(1, B.shape[0]), beta,
                                           _ptr(C), max(1, m)))
         return C
+
+    def sym_lowest(self, A, k: int):
+        """(w, Z) of the k lowest eigenpairs of a symmetric matrix of at most 192 rows,
+        k <= 32 (stda_hip_sym_lowest), or None when its eigenvalues lie too close."""
+        A = np.asfortranarray(A, dtype=np.float64)
+        n = A.shape[0]
+        w, Z, ok = np.zeros(k), np.zeros((n, k), order="F"), ctypes.c_int32()
+        self._check(self._L.stda_hip_sym_lowest(self._h, n, k, _ptr(A), _ptr(w), _ptr(Z),
+                                                ctypes.byref(ok)))
+        return (w, Z) if ok.value else None
 
     def kernel_stats(self, name: str):
         ms, n, w = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()

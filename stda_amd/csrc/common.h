@@ -245,6 +245,27 @@ void launch_tsgemm_nn2(hipStream_t s, int64_t n, int m, int p, double alpha, con
                        const double *A1, int64_t lda, const double *C, int64_t ldc, double beta,
                        double *out0, double *out1, int64_t ldo, const double *skip = nullptr);
 
+// --- Rayleigh-Ritz step (subspace.hip) ---------------------------------------------------
+// The k lowest eigenpairs of the live part of the symmetric subspace matrix of
+// m0 + mnew <= RR_MMAX columns, k <= RR_KMAX, one work-group.  H (ld ldh) holds
+// the matrix of the first m0 columns and receives the whole one; `gram` is the
+// new columns' block V^T A V(:, m0:) ((m0 + mnew) x mnew).
+constexpr int RR_MMAX = 192, RR_KMAX = 32;
+struct RRArgs {
+    int m0, mnew, k, ldh;
+    int restart;            // 1: the first m0 columns are Ritz vectors (H = diag(theta), live)
+    double *H;
+    const double *gram;
+    const double *flags;    // mnew, 0.0 for a dead new column; null: all live
+    int *alive;             // of the first m0 columns; receives those of all
+    double *refl;           // scratch, RR_MMAX * RR_MMAX
+    double *Y;              // out: (m0 + mnew) x min(k, m0 + mnew), min(k, live) of them
+                            // eigenvectors, zero in dead rows and further columns
+    double *theta;          // in (restart): Ritz values; out: min(k, live) ascending, then zeros
+    double *info;           // out: ok (0: eigenvalues too close or not finite), live, live new, 0
+};
+void launch_rr_lowest(hipStream_t s, const RRArgs &a);
+
 // --- batched Davidson (batch.hip): molecules in lock step ------------------------------
 constexpr int BATCH_MD = 64;                        // subspace limit
 constexpr int BATCH_KMAX = 24;                      // roots per molecule

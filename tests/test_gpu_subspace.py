@@ -1,0 +1,65 @@
+"""The subspace eigenkernel (stda_hip_sym_lowest) against numpy's eigh."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(float).eps
+
+
+@pytest.fixture(scope="module")
+def h():
+    from stda_amd.core import StdaHip
+    with StdaHip(0) as ctx:
+        yield ctx
+
+
+def matrix(kind, n, rng):
+    G = rng.standard_normal((n, n))
+    if kind == "dense":
+        return G + G.T
+    if kind == "davidson":      # a subspace matrix: rising diagonal, weak couplings
+        return np.diag(np.sort(rng.uniform(0.15, 0.5, n))) + 2e-3 * (G + G.T)
+    if kind == "ritz":          # after a restart: diagonal head, coupled tail
+        A = np.diag(np.sort(rng.uniform(0.15, 0.5, n)))
+        b = max(1, n // 4)
+        A[:, n - b:] += 1e-3 * G[:, n - b:]
+        A[n - b:, :] = A[:, n - b:].T
+        return 0.5 * (A + A.T)
+    Q = np.linalg.qr(G)[0]      # "close": pairs 1e-9 apart, orthogonal to 1e-7 only as they come
+    w = np.sort(rng.uniform(0.1, 1.0, n))
+    w[1::2] = w[:-1:2][:len(w[1::2])] + 1e-9
+    return (Q * w) @ Q.T
+
+
+@pytest.mark.parametrize("kind", ["dense", "davidson", "ritz", "close"])
+@pytest.mark.parametrize("n", [1, 2, 3, 8, 15, 16, 17, 32, 33, 63, 64, 65, 95, 96, 97, 120, 128,
+                               129, 160, 191, 192])
+def test_lowest_pairs(h, kind, n):
+    rng = np.random.default_rng(1000 * n + len(kind))
+    A = matrix(kind, n, rng)
+    A = 0.5 * (A + A.T)
+    norm = np.linalg.norm(A, 2)
+    for k in sorted({1, min(n, 20), min(n, 32)}):
+        out = h.sym_lowest(A, k)
+        assert out is not None
+        w, Z = out
+        # backward stable reduction: n eps |A| with a small constant
+        assert np.abs(w - np.linalg.eigvalsh(A)[:k]).max() <= 4 * n * EPS * norm
+        assert np.abs(Z.T @ Z - np.eye(k)).max() <= 8 * n * EPS
+        # an orthonormalisation of vectors with overlaps up to 1e-6 mixes values 1e-9 apart
+        assert np.linalg.norm(A @ Z - Z * w, axis=0).max() <= 8 * n * EPS * norm + 1e-14
+
+
+@pytest.mark.parametrize("n", [4, 40, 100])
+def test_repeated_and_nonfinite(h, n):
+    """Repeated eigenvalues and NaN: pairs that hold, or None, and always an end."""
+    for A in (np.eye(n), np.zeros((n, n)), np.diag(np.r_[np.ones(n // 2), 2 * np.ones(n - n // 2)])):
+        out = h.sym_lowest(A, min(n, 20))
+        if out is not None:
+            w, Z = out
+            assert np.abs(A @ Z - Z * w).max() <= 8 * n * EPS
+            assert np.abs(Z.T @ Z - np.eye(len(w))).max() <= 8 * n * EPS
+    A = np.eye(n)
+    A[0, n - 1] = A[n - 1, 0] = np.nan
+    assert h.sym_lowest(A, 2) is None
