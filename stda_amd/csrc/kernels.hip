@@ -1403,8 +1403,8 @@ __global__ void col_norm_final_kernel(int nsl, int k, const double *part, double
 // dropped when its pivot (the squared norm of its part orthogonal to the kept
 // columns before it) is at most thr * ref[j * ref_stride] (thr when ref is
 // null); alive[j] = 1.0 for the kept columns, 0.0 for the dropped ones.
-// Thread i owns row i of the factor, then column i of its inverse (forward
-// substitution).  S is
+// Lane i of one wave owns row i of the factor, then column i of its inverse
+// (forward substitution).  S is
 // given through G ((m + nt) x nt, ld ldg) = [V T]^T T of directions T before
 // their projection T - V G[0:m, :] against orthonormal V: S = G[m:m+nt, :] -
 // G[0:m, :]^T G[0:m, :] is the Gram matrix of the projected block (m = 0:
@@ -1416,133 +1416,146 @@ __global__ void col_norm_final_kernel(int nsl, int k, const double *part, double
 // |t_j|, and column k of T LinvT carries at most that sum of them: at the
 // bound it stays below about 1e-13 and another projection of T LinvT against
 // V would change nothing that matters, so the caller may leave it out.
+// LDS operations of a wave complete in order: keeps the compiler from moving them
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// value of lane `lane` (uniform), in scalar registers
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// NT: registers of a row, nt <= NT
+template <int NT>
 __global__ __launch_bounds__(256) void chol_inv_kernel(int nt, const double *__restrict__ G, int m,
                                                        int ldg, const double *__restrict__ ref,
                                                        int ref_stride, double thr,
                                                        double *__restrict__ LinvT,
                                                        double *__restrict__ alive,
                                                        double *__restrict__ skip) {
-    // L and Z (the inverse factor) share one buffer, which first holds the
-    // staged rows of G
+    // holds the staged rows of G, then S
     constexpr int SBUF = 2 * 64 * 65;
     __shared__ double buf[SBUF];
-    double *L = buf, *Z = buf + 64 * 65;
-    __shared__ int keep[64];
-    __shared__ double dg[64], lim[64];
+    double *L = buf;
     const int tid = threadIdx.x;
-    if (tid < nt) lim[tid] = thr * (ref ? ref[(int64_t)tid * ref_stride] : 1.0);
     // S = G[m:m+nt, :] - G[0:m, :]^T G[0:m, :]: the correction over chunks of
-    // SBUF / (nt + 1) rows of G (all of them for m <= 395 at nt = 20), loaded
-    // eight per thread before any is stored, each thread owning up to 16
-    // elements of S
+    // SBUF / (nt + 1) rows of G (all of them for m <= 395 at nt = 20); a wave
+    // loads whole columns
     const int ld = nt + 1, rows_per = SBUF / ld;
-    double acc[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) acc[u] = 0.0;
+    const int lane = tid & 63, wave = tid >> 6;
+    constexpr int NR = (NT + 15) / 16;   // elements (r16 + 16 a, c16 + 16 b) of S per thread
+    const int r16 = tid & 15, c16 = tid >> 4;
+    double acc[NR][NR] = {};
     for (int q0 = 0; q0 < m; q0 += rows_per) {
-        const int mq = min(rows_per, m - q0), tot = mq * nt;
+        const int mq = min(rows_per, m - q0);
         __syncthreads();
-        for (int e0 = 0; e0 < tot; e0 += 256 * 8) {
-            double v[8];
+        for (int c = wave; c < nt; c += 4) {
+            const double *g = G + q0 + (int64_t)ldg * c;
+            for (int q = lane; q < mq; q += 256) {   // four loads before any is stored
+                double v[4];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = e0 + tid + 256 * u;
-                v[u] = e < tot ? G[(q0 + e % mq) + (int64_t)ldg * (e / mq)] : 0.0;
-            }
+                for (int u = 0; u < 4; ++u) v[u] = q + 64 * u < mq ? g[q + 64 * u] : 0.0;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = e0 + tid + 256 * u;
-                if (e < tot) buf[(e % mq) * ld + e / mq] = v[u];
+                for (int u = 0; u < 4; ++u)
+                    if (q + 64 * u < mq) buf[(q + 64 * u) * ld + c] = v[u];
             }
         }
         __syncthreads();
+        int ro[NR], co[NR];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int e = tid + 256 * u;
-            if (e < nt * nt) {
-                const int r = e % nt, c = e / nt;
-                double s = 0.0;
-                for (int q = 0; q < mq; ++q) s += buf[q * ld + r] * buf[q * ld + c];
-                acc[u] -= s;
+        for (int a = 0; a < NR; ++a) {
+            ro[a] = min(r16 + 16 * a, nt - 1);
+            co[a] = min(c16 + 16 * a, nt - 1);
+        }
+#pragma unroll 2
+        for (int q = 0; q < mq; ++q) {
+            double x[NR], y[NR];
+#pragma unroll
+            for (int a = 0; a < NR; ++a) {
+                x[a] = buf[q * ld + ro[a]];
+                y[a] = buf[q * ld + co[a]];
             }
+#pragma unroll
+            for (int a = 0; a < NR; ++a)
+#pragma unroll
+                for (int b = 0; b < NR; ++b) acc[a][b] = fma(-x[a], y[b], acc[a][b]);
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int e = tid + 256 * u;
-        if (e < nt * nt) {
-            const int r = e % nt, c = e / nt;
-            L[r * 65 + c] = G[(m + r) + (int64_t)ldg * c] + acc[u];
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NR; ++b) {
+            const int r = r16 + 16 * a, c = c16 + 16 * b;
+            if (r < nt && c < nt) L[r * 65 + c] = G[(m + r) + (int64_t)ldg * c] + acc[a][b];
+        }
+    __syncthreads();
+    if (wave != 0) return;
+    // One wave factors and inverts in registers: lane i holds row i, a column of
+    // the factor reaches the other lanes as scalars (readlane).  Four waves with
+    // the matrix in LDS took two barriers a column: 24 us for the kernel at
+    // nt = 20 and m = 100, 31 us for one wave on LDS; 16 us this way, 9 us for
+    // nt <= 16.  The code is straight and read once, so a size has a kernel
+    // with no more of it than it needs.
+    double row[NT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) row[k] = lane < nt && k < nt ? L[lane * 65 + k] : 0.0;
+    const double lim = lane < nt ? thr * (ref ? ref[(int64_t)lane * ref_stride] : 1.0) : 0.0;
+    double rd = 0.0;                  // 1 / pivot of this lane's column, 0 when dropped
+    // Right-looking factor: step j takes the pivot, scales column j and
+    // subtracts l_ij l_kj from the columns k > j
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {   // rows and columns from nt on are zero: dropped
+        const double d = lane_value(row[j], j);
+        if (d > lane_value(lim, j) && d > 0.0) {
+            const double r = 1.0 / sqrt(d);
+            const double l = lane > j ? row[j] * r : 0.0;
+            row[j] = l;
+            if (lane == j) rd = r;
+#pragma unroll
+            for (int k = j + 1; k < NT; ++k) row[k] = fma(-l, lane_value(l, k), row[k]);
+        } else {
+            row[j] = 0.0;
         }
     }
-    __syncthreads();
-    // Right-looking factor, one barrier per step: step j takes the pivot of
-    // column j and subtracts l_ij l_kj (l = column j over its root, formed
-    // where it is used) from the trailing lower triangle; column j itself is
-    // scaled in step j + 1, when nothing reads it.  Every element sees the
-    // same operations in the same order as in the left-looking form.
-    for (int j = 0; j < nt; ++j) {
-        const double d = L[j * 65 + j];
-        const bool kp = d > lim[j] && d > 0.0;
-        const double ljj = kp ? sqrt(d) : 0.0;
-        if (j > 0 && tid >= j && tid < nt) {
-            const int pj = j - 1;
-            L[tid * 65 + pj] = keep[pj] ? L[tid * 65 + pj] / dg[pj] : 0.0;
-        }
-        if (tid == 0) {
-            keep[j] = kp ? 1 : 0;
-            dg[j] = ljj;
-        }
-        if (kp) {
-            const int w = nt - j - 1;
-            for (int e = tid; e < w * w; e += 256) {
-                const int i = j + 1 + e % w, k = j + 1 + e / w;
-                if (k <= i) L[i * 65 + k] -= (L[i * 65 + j] / ljj) * (L[k * 65 + j] / ljj);
+    // inverse on the kept indices by forward substitution: lane c holds column c
+    double z[NT];
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+        z[r] = 0.0;
+        const double dr = lane_value(rd, r);
+        if (dr != 0.0) {
+            double s0 = r == lane ? 1.0 : 0.0, s1 = 0.0;
+#pragma unroll
+            for (int k = 0; k < r; ++k) {
+                const double l = lane_value(row[k], r);
+                if (k & 1) s1 = fma(-l, z[k], s1);
+                else s0 = fma(-l, z[k], s0);
             }
+            z[r] = (s0 + s1) * dr;
         }
-        __syncthreads();
+        if (lane < nt && r < nt) LinvT[lane + nt * r] = z[r];
     }
-    if (tid < nt) L[tid * 65 + tid] = dg[tid];
-    // inverse on the kept indices, row by row (forward substitution over all
-    // columns at once): step r subtracts L_ir (row r over its pivot) from the
-    // rows below; row r is divided in step r + 1
-    for (int e = tid; e < nt * nt; e += 256) {
-        const int r = e / nt, q = e % nt;
-        Z[r * 65 + q] = (r == q && keep[r]) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    for (int r = 0; r < nt; ++r) {
-        if (r > 0 && tid < r && keep[r - 1] && keep[tid]) Z[(r - 1) * 65 + tid] /= dg[r - 1];
-        if (keep[r]) {
-            const double lrr = dg[r];
-            const int w = nt - r - 1, h = r + 1;
-            for (int e = tid; e < w * h; e += 256) {
-                const int i = r + 1 + e / h, q = e % h;
-                if (keep[i] && keep[q]) Z[i * 65 + q] -= L[i * 65 + r] * (Z[r * 65 + q] / lrr);
-            }
-        }
-        __syncthreads();
-    }
-    if (tid < nt && keep[nt - 1] && keep[tid]) Z[(nt - 1) * 65 + tid] /= dg[nt - 1];
-    __syncthreads();
-    for (int e = tid; e < nt * nt; e += 256) LinvT[e] = Z[(e / nt) * 65 + e % nt];
-    if (tid < nt) alive[tid] = keep[tid] ? 1.0 : 0.0;
+    if (lane < nt) alive[lane] = rd != 0.0 ? 1.0 : 0.0;
     if (skip && ref) {
-        // row k of Z holds the coefficients of column k of T LinvT; lim[]
-        // is no longer read, so it takes the row sums
-        if (tid < nt) {
-            double a = 0.0;
-            for (int j = 0; j <= tid; ++j)
-                a += fabs(Z[tid * 65 + j]) * sqrt(fmax(ref[(int64_t)j * ref_stride], 0.0));
-            lim[tid] = a;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double a = 0.0;
-            for (int k = 0; k < nt; ++k) a = fmax(a, lim[k]);
-            skip[0] = a <= 1.0e3 ? 1.0 : 0.0;   // NaN rows fail the test
-        }
+        // row k of the inverse holds the coefficients of column k of T LinvT;
+        // its sum goes through LDS, column by column
+        const double w = lane < nt ? sqrt(fmax(ref[(int64_t)lane * ref_stride], 0.0)) : 0.0;
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+            if (k < nt) buf[lane * 65 + k] = fabs(z[k]) * w;
+        wave_fence();
+        double a = 0.0;
+        if (lane < nt)
+            for (int j = 0; j < nt; ++j) a += buf[j * 65 + lane];
+        const bool small = a <= 1.0e3;   // NaN rows fail the test
+        const bool ok = __all(small);
+        if (lane == 0) skip[0] = ok ? 1.0 : 0.0;
     }
 }
 
@@ -1551,8 +1564,15 @@ void launch_chol_inv(hipStream_t s, int nt, const double *G, int m, int ldg, con
     if (nt <= 0) return;
     if (nt > 64) throw Error(STDA_HIP_ERR_ARG, "chol_inv: more than 64 columns");
     if (skip && !ref) throw Error(STDA_HIP_ERR_ARG, "chol_inv: the skip test needs the norms");
-    hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(256), 0, s, nt, G, m, ldg, ref, ref_stride,
-                       thr, LinvT, alive, skip);
+#define STDA_CHOL(NT)                                                                        \
+    hipLaunchKernelGGL((chol_inv_kernel<NT>), dim3(1), dim3(256), 0, s, nt, G, m, ldg, ref,      \
+                       ref_stride, thr, LinvT, alive, skip)
+    if (nt <= 16) STDA_CHOL(16);
+    else if (nt <= 24) STDA_CHOL(24);
+    else if (nt <= 32) STDA_CHOL(32);
+    else if (nt <= 48) STDA_CHOL(48);
+    else STDA_CHOL(64);
+#undef STDA_CHOL
 }
 
 void launch_col_norms_split(hipStream_t s, int64_t n, int k, const double *R, double *part,

@@ -81,7 +81,7 @@ struct RRSmem {
     double d[MX], e[MX], e2[MX], tau[MX];
     double f[MX * RR_LD];   // forward pivots, then the vectors Z
     double g[MX * RR_LD];   // backward pivots, then reflector chunks
-    double gram[RR_K * RR_LD];
+    double2 gram[RR_K * RR_K / 2];
     double lam[RR_K], lo[RR_K], hi[RR_K];
     double gam[RR_K];
     double red[16];
@@ -441,7 +441,7 @@ __global__ void __launch_bounds__(16 * RT, 1) rr_lowest_kernel(RRArgs p) {
             const double one = t == u ? 1.0 : 0.0;
             const double x = in ? fabs(acc[q] - one) : 0.0;
             dev = x > dev || !(x == x) ? x : dev;
-            sm.gram[t * RR_LD + u] = in ? 1.5 * one - 0.5 * acc[q] : 0.0;
+            reinterpret_cast<double *>(sm.gram)[t * RR_K + u] = in ? 1.5 * one - 0.5 * acc[q] : 0.0;
         }
         for (int o = 32; o > 0; o >>= 1) {
             const double x = __shfl_xor(dev, o, 64);
@@ -468,9 +468,13 @@ __global__ void __launch_bounds__(16 * RT, 1) rr_lowest_kernel(RRArgs p) {
             for (int u = 4 * part; u < kk; u += 4 * (T / 256)) {   // gram is zero beyond kk
                 double y[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int q = 0; q < RR_K; ++q)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) y[r] = fma(z[q], sm.gram[q * RR_LD + u + r], y[r]);
+                for (int q = 0; q < RR_K; ++q) {
+                    const double2 w0 = sm.gram[(q * RR_K + u) / 2], w1 = sm.gram[(q * RR_K + u) / 2 + 1];
+                    y[0] = fma(z[q], w0.x, y[0]);
+                    y[1] = fma(z[q], w0.y, y[1]);
+                    y[2] = fma(z[q], w1.x, y[2]);
+                    y[3] = fma(z[q], w1.y, y[3]);
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) sm.f[row * RR_LD + u + r] = y[r];
             }
