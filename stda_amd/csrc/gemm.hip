@@ -15,7 +15,7 @@
 //           FP32 accumulation (the lo lo term, ~2^-18 relative, is dropped).
 //
 // Work-group: 256 threads (four waves) own a BT x BT tile of C (BT = 128, or
-// 64 when the 128-tiles would leave compute units idle); wave w owns rows
+// 64 or 32 when the larger tiles would leave compute units idle); wave w owns rows
 // BT/2 (w / 2) .. + BT/2 and columns BT/2 (w % 2) .. + BT/2, i.e. (BT/32)^2
 // MFMA blocks of 16 x 16.  K advances in chunks (16 for F64/F32, 32 for BF16X3):
 // each thread loads its share of the next chunk into registers (coalesced
@@ -324,8 +324,12 @@ std::mutex g_tile_mu;
 std::map<TileKey, int> g_tile_choice;   // 0: being tuned
 
 int rule_tile(int M, int N, int batch) {
-    const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batch;
-    return big >= 512 ? 128 : 64;
+    auto tiles = [&](int bt) { return (int64_t)((M + bt - 1) / bt) * ((N + bt - 1) / bt) * batch; };
+    if (tiles(128) >= 512) return 128;
+    // A 64-tile holds its compute unit for 1024 cycles of FP64 MFMA per 16 rows of
+    // K: with fewer of them than compute units, 32-tiles (a quarter of that)
+    // spread the work
+    return tiles(64) >= 256 ? 64 : 32;
 }
 
 int ilog2(int64_t v) {
@@ -410,8 +414,10 @@ void launch_tile(hipStream_t s, int bt, bool ta, bool tb, int M, int N, int K, T
                            N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC);
     if (bt == 128) {
         STDA_GEMM_LAUNCH(128)
-    } else {
+    } else if (bt == 64) {
         STDA_GEMM_LAUNCH(64)
+    } else {
+        STDA_GEMM_LAUNCH(32)
     }
 #undef STDA_GEMM_LAUNCH
     STDA_HIP_CHECK(hipGetLastError());

@@ -63,3 +63,38 @@ def test_repeated_and_nonfinite(h, n):
     A = np.eye(n)
     A[0, n - 1] = A[n - 1, 0] = np.nan
     assert h.sym_lowest(A, 2) is None
+
+
+@pytest.mark.parametrize("k", [1, 3, 10, 16, 17, 20, 24, 25, 32, 33, 48, 49, 64])
+def test_root_counts(h, k):
+    """The k lowest roots for block widths on both sides of every kernel size (block
+    orthonormalisation, subspace step) against the dense eigenvalues of the explicit A."""
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    if not hasattr(test_root_counts, "ref"):
+        mol, ints = cluster(24, seed=11, basis="minimal")
+        ci = prepare(mol, 7.0, 0.25, ints)
+        h.setup(ci, 7.0, 0.25)
+        test_root_counts.ref = ci, np.linalg.eigvalsh(h.build_a())
+    ci, w = test_root_counts.ref
+    h.setup(ci, 7.0, 0.25)
+    sol = h.solve_tda(k)
+    assert len(sol.omega) == k
+    # residual norms of 1e-8 bound the roots by 1e-8, and squared over the gap in practice
+    assert np.abs(sol.omega - w[:k]).max() <= 1e-10
+    assert np.abs(sol.X.T @ sol.X - np.eye(k)).max() <= 1e-11
+
+
+@pytest.mark.parametrize("mode,unit", [("fp64", EPS), ("fp32", 2.0 ** -24)])
+@pytest.mark.parametrize("m,n,kk", [(33, 31, 50), (320, 330, 37), (1030, 1050, 37), (2950, 2890, 19)])
+def test_gemm_tile_sizes(h, mode, unit, m, n, kk):
+    """Shapes of each tile size of the matrix-core GEMM (32, 32, 64, 128), ragged edges."""
+    rng = np.random.default_rng(m)
+    A, B = rng.standard_normal((m, kk)), rng.standard_normal((kk, n))
+    if mode == "fp32":
+        A, B = A.astype(np.float32).astype(float), B.astype(np.float32).astype(float)
+    for ta in (False, True):
+        for tb in (False, True):
+            C = h.gemm(A.T if ta else A, B.T if tb else B, ta=ta, tb=tb, mode=mode)
+            bound = (kk + 2) * unit * (np.abs(A) @ np.abs(B))
+            assert (np.abs(C - A @ B) <= bound + kk * EPS).all()
