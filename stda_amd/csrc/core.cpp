@@ -80,7 +80,12 @@ using dpotrf_t = void (*)(const char *, const int *, double *, const int *, int 
 using dtrsm_t = void (*)(const char *, const char *, const char *, const char *, const int *,
                          const int *, const double *, const double *, const int *, double *,
                          const int *);
+using dpotri_t = void (*)(const char *, const int *, double *, const int *, int *);
+using dsysv_t = void (*)(const char *, const int *, const int *, double *, const int *, int *,
+                         double *, const int *, double *, const int *, int *);
 struct HostLapack {
+    dpotri_t potri = nullptr;
+    dsysv_t sysv = nullptr;
     dsyevd_t syevd = nullptr;
     dgemm_t gemm = nullptr;
     dpotrf_t potrf = nullptr;
@@ -102,6 +107,8 @@ static HostLapack find_lapack() {
         L.gemm = (dgemm_t)dlsym(h, "dgemm_");
         L.potrf = (dpotrf_t)dlsym(h, "dpotrf_");
         L.trsm = (dtrsm_t)dlsym(h, "dtrsm_");
+        L.potri = (dpotri_t)dlsym(h, "dpotri_");
+        L.sysv = (dsysv_t)dlsym(h, "dsysv_");
         break;
     }
     return L;
@@ -300,6 +307,41 @@ void host_solve_lt(int n, int k, const std::vector<double> &L, double *B, int ld
     }
 }
 
+// B(n x k) <- (L L^T)^-1 B; false without LAPACK.
+bool host_potrs(int n, int k, const std::vector<double> &L, double *B, int ldb) {
+    auto fn = host_lapack().trsm;
+    if (!fn) return false;
+    const double one = 1.0;
+    fn("L", "L", "N", "N", &n, &k, &one, L.data(), &n, B, &ldb);
+    fn("L", "L", "T", "N", &n, &k, &one, L.data(), &n, B, &ldb);
+    return true;
+}
+
+// Inverse of the symmetric positive definite L L^T from its lower factor (both
+// triangles filled); false without LAPACK.
+bool host_potri(int n, std::vector<double> &a) {
+    auto fn = host_lapack().potri;
+    if (!fn) return false;
+    int info = 0;
+    fn("L", &n, a.data(), &n, &info);
+    if (info != 0) return false;
+    for (int j = 1; j < n; ++j)
+        for (int i = 0; i < j; ++i) a[i + (size_t)n * j] = a[j + (size_t)n * i];
+    return true;
+}
+
+// B(n x k) <- A^-1 B for a symmetric, possibly indefinite A (destroyed):
+// Bunch-Kaufman factorisation; false when it breaks down or without LAPACK.
+bool host_sysv(int n, int k, std::vector<double> &a, double *B, int ldb) {
+    auto fn = host_lapack().sysv;
+    if (!fn) return false;
+    int info = 0, lwork = 64 * n;
+    std::vector<int> piv(n);
+    std::vector<double> work(lwork);
+    fn("L", &n, &k, a.data(), &n, piv.data(), B, &ldb, work.data(), &lwork, &info);
+    return info == 0;
+}
+
 struct Timer {
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
     double ms() const {
@@ -476,6 +518,7 @@ struct stda_hip_ctx {
             STDA_HIP_CHECK(hipStreamSynchronize(stream));
             if (pin) (void)hipHostFree(pin);
             pin = nullptr;
+            n = std::max(n, 2 * pin_n);   // growing spaces ask for a little more each time
             pin_n = 0;
             STDA_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), n * sizeof(double), 0));
             pin_n = n;
@@ -859,34 +902,6 @@ void apply_ops(stda_hip_ctx *c, int op1, int op2, int nvec, const double *V, int
 
 // ------------------------------------------------------------------------------------------
 // small dense helpers (host)
-std::vector<double> sym_sqrt(const std::vector<double> &A, int m, bool inverse, double *minev) {
-    std::vector<double> U(A), w;
-    host_syev(m, U, w);
-    if (minev) *minev = m ? w[0] : 0.0;
-    std::vector<double> R((size_t)m * m, 0.0);
-    for (int k = 0; k < m; ++k) {
-        double f = w[k] > 0 ? std::sqrt(w[k]) : 0.0;
-        if (inverse) f = f > 0 ? 1.0 / f : 0.0;
-        for (int j = 0; j < m; ++j) {
-            double ujk = U[j + (size_t)m * k] * f;
-            for (int i = 0; i < m; ++i) R[i + (size_t)m * j] += U[i + (size_t)m * k] * ujk;
-        }
-    }
-    return R;
-}
-
-std::vector<double> matmul(const std::vector<double> &A, const std::vector<double> &B, int m,
-                           int k, int n) {   // (m x k)(k x n), column-major
-    std::vector<double> C((size_t)m * n, 0.0);
-    for (int j = 0; j < n; ++j)
-        for (int l = 0; l < k; ++l) {
-            double b = B[l + (size_t)k * j];
-            if (b == 0.0) continue;
-            for (int i = 0; i < m; ++i) C[i + (size_t)m * j] += A[i + (size_t)m * l] * b;
-        }
-    return C;
-}
-
 // Orthonormalise the columns of T (n x nt, device) against V (n x m, device,
 // orthonormal) and among themselves; returns the number of columns kept,
 // packed at the front of T.
@@ -1019,6 +1034,10 @@ struct DavOpts {
     int nv0 = 0;
     int maxiter = 300;
     bool allow_unconverged = false;
+    // Every root up to this value is wanted (0: the k roots asked for): the solver
+    // returns as soon as k Ritz values lie within it.  They bound the roots from
+    // above, so k roots are too few and iterating them further is in vain.
+    double window = 0.0;
 };
 
 void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta,
@@ -1198,6 +1217,7 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
         }
         m = mt;
         const double *th = devrr ? nrm + k : yt.get() + (size_t)m * kk;
+        if (o.window > 0.0 && kk == k && k < n && theta[k - 1] <= o.window) return;
         std::vector<int> un;
         for (int j = 0; j < kk; ++j)
             if (!(rn[j] < tol)) un.push_back(j);
@@ -1259,15 +1279,42 @@ void davidson_rpa(stda_hip_ctx *c, int k, double tol, std::vector<double> &omega
     const int kt_max = (int)std::min<int64_t>(n, k + std::max(8, k / 2));
     int maxdim = (int)std::min<int64_t>(n, std::max(10 * k, 2 * k + 128));
     if (maxdim < nguess) maxdim = nguess;
+    const int bmax = std::max({nguess, 2 * k, std::min(o.nv0, maxdim)});   // columns of a new block
+    const bool devortho = 2 * k <= 64;   // new blocks orthonormalised without a host round trip
     DBuf<double> V((size_t)n * maxdim), P((size_t)n * maxdim), M((size_t)n * maxdim);
-    DBuf<double> R((size_t)n * 2 * k), PX((size_t)n * k), MX((size_t)n * k), tmp, Yd, nrm(2 * k);
+    DBuf<double> R((size_t)n * 2 * k), PX((size_t)n * k), MX((size_t)n * k), tmp, nrm(2 * k);
+    // Gram blocks of A+B and A-B and the alive flags of the new block (one
+    // download); coefficients of X+Y and X-Y and the frequencies, twice (one upload)
+    DBuf<double> Hc((size_t)2 * maxdim * bmax + bmax), Yd((size_t)2 * maxdim * k + 2 * k), T2, ow, rr;
+    DBuf<int> lived;
+    if (devortho) {
+        T2.resize((size_t)n * 2 * k);
+        ow.resize(3 * (size_t)(maxdim + 2 * k) * 2 * k + (size_t)4 * k * k + 1);
+    }
+    const size_t rrz = (size_t)RR_MMAX * RR_KMAX + RR_KMAX + 4;   // vectors, values, report
+    if (kt_max <= RR_KMAX) {
+        rr.resize(rrz + 3 * (size_t)RR_MMAX * RR_MMAX);
+        lived.resize(RR_MMAX);
+    }
     XpY.resize((size_t)n * k);
     XmY.resize((size_t)n * k);
+    const size_t o_hc = 0, o_y = o_hc + (size_t)2 * maxdim * bmax + bmax,
+                 o_rn = o_y + (size_t)2 * maxdim * k + 2 * k, o_z = o_rn + 2 * (size_t)k,
+                 o_h = o_z + rrz;
+    double *pin = c->pinned(o_h + (size_t)RR_MMAX * RR_MMAX);
     int m = 0, mnew = nguess;
+    bool flags_pending = false;
     if (o.V0) {
         int nv0 = std::min(o.nv0, maxdim);
         STDA_HIP_CHECK(hipMemcpyAsync(V.get(), o.V0, (size_t)n * nv0 * 8, hipMemcpyDeviceToDevice, s));
-        mnew = orthonormalize(c, V.get(), 0, V.get(), nv0, tmp);
+        if (devortho && nv0 <= 2 * k) {
+            mnew = nv0;
+            orthonormalize_dev(c, V.get(), 0, V.get(), nv0, T2.get(), ow.get(),
+                               Hc.get() + (size_t)2 * nv0 * nv0);
+            flags_pending = true;
+        } else {
+            mnew = orthonormalize(c, V.get(), 0, V.get(), nv0, tmp);
+        }
     } else {
         std::vector<int32_t> rows = lowest_diag_rows(c->ed_h, nguess);
         DBuf<int32_t> rowsd;
@@ -1275,123 +1322,149 @@ void davidson_rpa(stda_hip_ctx *c, int k, double tol, std::vector<double> &omega
         launch_set_unit(s, n, nguess, V.get(), rowsd.get());
     }
     std::vector<double> Ap((size_t)maxdim * maxdim, 0.0), Am((size_t)maxdim * maxdim, 0.0);
+    std::vector<double> ap, L, t1, Hm, w2, Z, xt, at;
+    auto no_progress = [&]() {   // every new direction lies in the space already
+        if (o.allow_unconverged) return;
+        throw Error(STDA_HIP_ERR_NOT_CONVERGED, "RPA Davidson did not converge (no new directions)");
+    };
     for (int it = 0; it < o.maxiter; ++it) {
         apply_ops(c, OP_APB, OP_AMB, mnew, V.get() + n * m, n, P.get() + n * m, n, M.get() + n * m,
                   n, o.fp32);
         int mt = m + mnew;
-        DBuf<double> Hc((size_t)mt * mnew * 2);
+        const size_t blk = (size_t)mt * mnew;
         dgemm_tn(c, mt, mnew, n, V.get(), n, P.get() + n * m, n, Hc.get());
-        dgemm_tn(c, mt, mnew, n, V.get(), n, M.get() + n * m, n, Hc.get() + (size_t)mt * mnew);
-        std::vector<double> hc((size_t)mt * mnew * 2);
-        Hc.download(hc.data(), hc.size(), s);
+        dgemm_tn(c, mt, mnew, n, V.get(), n, M.get() + n * m, n, Hc.get() + blk);
+        double *hc = pin + o_hc;
+        STDA_HIP_CHECK(hipMemcpyAsync(hc, Hc.get(), (2 * blk + (flags_pending ? mnew : 0)) * 8,
+                                      hipMemcpyDeviceToHost, s));
         c->sync();
+        // columns of the new block that brought nothing (zero) leave the space
+        std::vector<int> keep;
         for (int j = 0; j < mnew; ++j)
-            for (int i = 0; i < mt; ++i) {
-                double vp = hc[i + (size_t)mt * j], vm = hc[(size_t)mt * mnew + i + (size_t)mt * j];
+            if (!flags_pending || hc[2 * blk + j] != 0.0) keep.push_back(j);
+        flags_pending = false;
+        if (keep.empty()) { no_progress(); return; }
+        const int nk = (int)keep.size();
+        for (int j = 0; j < nk; ++j) {
+            const int cj = keep[j];
+            if (cj != j)
+                for (DBuf<double> *B : {&V, &P, &M})
+                    STDA_HIP_CHECK(hipMemcpyAsync(B->get() + n * (m + j), B->get() + n * (m + cj),
+                                                  (size_t)n * 8, hipMemcpyDeviceToDevice, s));
+            for (int i = 0; i < m + nk; ++i) {
+                const int ci = i < m ? i : m + keep[i - m];
+                const double vp = hc[ci + (size_t)mt * cj], vm = hc[blk + ci + (size_t)mt * cj];
                 Ap[i + (size_t)maxdim * (m + j)] = vp; Ap[(m + j) + (size_t)maxdim * i] = vp;
                 Am[i + (size_t)maxdim * (m + j)] = vm; Am[(m + j) + (size_t)maxdim * i] = vm;
             }
-        m = mt;
-        std::vector<double> ap((size_t)m * m), am((size_t)m * m);
+        }
+        m += nk;
+        // Reduced problem with A-B = L L^T: L^T (A+B) L z = w^2 z, X+Y = L z
+        // (its Hermitian square root took two eigenproblems and three times the
+        // products; written as loops they were most of an RPA solve)
+        ap.resize((size_t)m * m);
+        L.resize((size_t)m * m);
+        t1.resize((size_t)m * m);
+        Hm.resize((size_t)m * m);
         for (int j = 0; j < m; ++j)
             for (int i = 0; i < m; ++i) {
                 ap[i + (size_t)m * j] = 0.5 * (Ap[i + (size_t)maxdim * j] + Ap[j + (size_t)maxdim * i]);
-                am[i + (size_t)m * j] = 0.5 * (Am[i + (size_t)maxdim * j] + Am[j + (size_t)maxdim * i]);
+                L[i + (size_t)m * j] = 0.5 * (Am[i + (size_t)maxdim * j] + Am[j + (size_t)maxdim * i]);
             }
-        double minev = 0.0;
-        std::vector<double> sq = sym_sqrt(am, m, false, &minev);
-        if (minev <= 0.0)
+        if (!host_potrf_lower(m, L))
             throw Error(STDA_HIP_ERR_AMB_NOT_PD, "matrix power impossible (A-B not positive definite)");
-        std::vector<double> Hm = matmul(matmul(sq, ap, m, m, m), sq, m, m, m), w2;
-        host_syev(m, Hm, w2);
-        int kk = std::min(k, m);
-        omega.assign(kk, 0.0);
-        std::vector<double> xr((size_t)m * kk), yr((size_t)m * kk);   // (X+Y)_red, (X-Y)_red
-        std::vector<double> Z(Hm.begin(), Hm.begin() + (size_t)m * kk);
-        std::vector<double> xp = matmul(sq, Z, m, m, kk);
-        for (int j = 0; j < kk; ++j) {
-            if (w2[j] <= 0.0) throw Error(STDA_HIP_ERR_NO_ROOTS, "RPA diag failed (w^2 <= 0)");
-            omega[j] = std::sqrt(w2[j]);
-            double f = 1.0 / std::sqrt(omega[j]);
-            for (int i = 0; i < m; ++i) xr[i + (size_t)m * j] = xp[i + (size_t)m * j] * f;
+        host_gemm(false, false, m, m, m, 1.0, ap.data(), m, L.data(), m, 0.0, t1.data(), m);
+        host_gemm(true, false, m, m, m, 1.0, L.data(), m, t1.data(), m, 0.0, Hm.data(), m);
+        const int kt = std::min(m, kt_max), kk = std::min(k, m);
+        bool have = false;
+        if (m <= RR_MMAX && kt <= RR_KMAX) {   // the lowest kt pairs on the device
+            double *zd = rr.get(), *hd = zd + rrz;
+            std::copy(Hm.begin(), Hm.end(), pin + o_h);
+            STDA_HIP_CHECK(hipMemcpyAsync(hd, pin + o_h, (size_t)m * m * 8, hipMemcpyHostToDevice, s));
+            RRArgs ra{};
+            ra.mnew = m;
+            ra.k = kt;
+            ra.ldh = m;
+            ra.H = hd + (size_t)RR_MMAX * RR_MMAX;
+            ra.gram = hd;
+            ra.alive = lived.get();
+            ra.refl = hd + 2 * (size_t)RR_MMAX * RR_MMAX;
+            ra.Y = zd;
+            ra.theta = zd + (size_t)m * kt;
+            ra.info = zd + (size_t)m * kt + kt;
+            launch_rr_lowest(s, ra);
+            STDA_HIP_CHECK(hipMemcpyAsync(pin + o_z, zd, ((size_t)m * kt + kt + 4) * 8,
+                                          hipMemcpyDeviceToHost, s));
+            c->sync();
+            const double *z = pin + o_z;
+            have = z[(size_t)m * kt + kt] != 0.0;
+            if (have) {
+                Z.assign(z, z + (size_t)m * kt);
+                w2.assign(z + (size_t)m * kt, z + (size_t)m * kt + kt);
+            }
         }
-        std::vector<double> apx = matmul(ap, xr, m, m, kk);
-        for (int j = 0; j < kk; ++j)
-            for (int i = 0; i < m; ++i) yr[i + (size_t)m * j] = apx[i + (size_t)m * j] / omega[j];
+        if (!have) {
+            host_syev(m, Hm, w2);
+            Z.assign(Hm.begin(), Hm.begin() + (size_t)m * kt);
+        }
+        // (X+Y)_red = L z / sqrt(w), (X-Y)_red = (A+B) (X+Y)_red / w
+        xt.resize((size_t)m * kt);
+        at.resize((size_t)m * kt);
+        host_gemm(false, false, m, kt, m, 1.0, L.data(), m, Z.data(), m, 0.0, xt.data(), m);
+        omega.assign(kk, 0.0);
+        for (int j = 0; j < kt; ++j) {
+            if (j < kk) {
+                if (w2[j] <= 0.0) throw Error(STDA_HIP_ERR_NO_ROOTS, "RPA diag failed (w^2 <= 0)");
+                omega[j] = std::sqrt(w2[j]);
+            }
+            const double f = 1.0 / std::sqrt(std::sqrt(std::max(w2[j], 1.0e-300)));
+            for (int i = 0; i < m; ++i) xt[i + (size_t)m * j] *= f;
+        }
+        host_gemm(false, false, m, kt, m, 1.0, ap.data(), m, xt.data(), m, 0.0, at.data(), m);
+        for (int j = 0; j < kt; ++j) {
+            const double f = 1.0 / std::sqrt(std::max(w2[j], 1.0e-300));
+            for (int i = 0; i < m; ++i) at[i + (size_t)m * j] *= f;
+        }
         // full-space Ritz vectors and residuals
-        std::vector<double> both((size_t)m * 2 * kk);
-        std::copy(xr.begin(), xr.end(), both.begin());
-        std::copy(yr.begin(), yr.end(), both.begin() + (size_t)m * kk);
-        Yd.upload(both.data(), both.size(), s);
-        gemm_nn(c, n, kk, m, 1.0, V.get(), n, Yd.get(), m, 0.0, XpY.get(), n);
-        gemm_nn(c, n, kk, m, 1.0, V.get(), n, Yd.get() + (size_t)m * kk, m, 0.0,
-              XmY.get(), n);
-        gemm_nn(c, n, kk, m, 1.0, P.get(), n, Yd.get(), m, 0.0, PX.get(), n);
-        gemm_nn(c, n, kk, m, 1.0, M.get(), n, Yd.get() + (size_t)m * kk, m, 0.0,
-              MX.get(), n);
-        DBuf<double> om;
-        om.upload(omega.data(), kk, s);
-        launch_residual(s, n, kk, PX.get(), XmY.get(), om.get(), R.get());            // (A+B)(X+Y) - w(X-Y)
-        launch_residual(s, n, kk, MX.get(), XpY.get(), om.get(), R.get() + n * kk);   // (A-B)(X-Y) - w(X+Y)
-        col_norms(c, n, 2 * kk, R.get(), nrm.get());
-        std::vector<double> rn(2 * kk);
-        nrm.download(rn.data(), 2 * kk, s);
+        const size_t mk = (size_t)m * kk;
+        double *Yh = pin + o_y;
+        std::copy(xt.begin(), xt.begin() + mk, Yh);
+        std::copy(at.begin(), at.begin() + mk, Yh + mk);
+        for (int q = 0; q < 2; ++q) std::copy(omega.begin(), omega.end(), Yh + 2 * mk + q * kk);
+        STDA_HIP_CHECK(hipMemcpyAsync(Yd.get(), Yh, (2 * mk + 2 * kk) * 8, hipMemcpyHostToDevice, s));
+        const double *om = Yd.get() + 2 * mk;
+        gemm_nn2(c, n, kk, m, V.get(), P.get(), n, Yd.get(), m, XpY.get(), PX.get(), n);
+        gemm_nn2(c, n, kk, m, V.get(), M.get(), n, Yd.get() + mk, m, XmY.get(), MX.get(), n);
+        residual_norms(c, n, kk, PX.get(), XmY.get(), om, R.get(), nrm.get());   // (A+B)(X+Y) - w(X-Y)
+        residual_norms(c, n, kk, MX.get(), XpY.get(), om, R.get() + n * kk,      // (A-B)(X-Y) - w(X+Y)
+                       nrm.get() + kk);
+        double *rn = pin + o_rn;
+        STDA_HIP_CHECK(hipMemcpyAsync(rn, nrm.get(), (size_t)2 * kk * 8, hipMemcpyDeviceToHost, s));
         c->sync();
-        std::vector<int> un;
-        for (int j = 0; j < 2 * kk; ++j)
-            if (!(rn[j] < tol)) un.push_back(j);
-        if (un.empty() && kk == k) return;
+        if (o.window > 0.0 && kk == k && k < n && omega[k - 1] <= o.window) return;
+        int nun = 0;
+        for (int j = 0; j < 2 * kk; ++j) nun += !(rn[j] < tol);
+        if (nun == 0 && kk == k) return;
         if (m == n) return;
         if (it + 1 == o.maxiter && o.allow_unconverged) return;
-        int nun = (int)un.size();
-        for (int q = 0; q < nun; ++q)
-            if (un[q] != q)
-                STDA_HIP_CHECK(hipMemcpyAsync(R.get() + n * q, R.get() + n * un[q], n * 8,
-                                              hipMemcpyDeviceToDevice, s));
-        std::vector<double> thu(nun);
-        for (int q = 0; q < nun; ++q) thu[q] = omega[un[q] % kk];
-        DBuf<double> thud;
-        thud.upload(thu.data(), nun, s);
-        launch_precondition(s, n, nun, R.get(), c->ed.get(), thud.get(), R.get());
         if (m + nun > maxdim) {
             // restart: V <- orthonormal basis of span(X+Y, X-Y) of the lowest kt
             // Ritz pairs, P/M transformed alike
-            const int kt = std::min(m, kt_max);
-            std::vector<double> G((size_t)m * 2 * kt);
-            {
-                std::vector<double> Zt(Hm.begin(), Hm.begin() + (size_t)m * kt);
-                std::vector<double> xt = matmul(sq, Zt, m, m, kt);
-                for (int j = 0; j < kt; ++j) {
-                    const double wj = std::sqrt(std::max(w2[j], 1.0e-300));
-                    for (int i = 0; i < m; ++i) xt[i + (size_t)m * j] /= std::sqrt(wj);
-                }
-                std::vector<double> at = matmul(ap, xt, m, m, kt);
-                for (int j = 0; j < kt; ++j) {
-                    const double wj = std::sqrt(std::max(w2[j], 1.0e-300));
-                    for (int i = 0; i < m; ++i) {
-                        G[i + (size_t)m * j] = xt[i + (size_t)m * j];
-                        G[i + (size_t)m * (kt + j)] = at[i + (size_t)m * j] / wj;
-                    }
-                }
-            }
-            int nc = 2 * kt;
-            std::vector<double> S = matmul([&] {
-                std::vector<double> t((size_t)nc * m);
-                for (int j = 0; j < nc; ++j)
-                    for (int i = 0; i < m; ++i) t[j + (size_t)nc * i] = G[i + (size_t)m * j];
-                return t;
-            }(), G, nc, m, nc), w;
+            const int nc = 2 * kt;
+            std::vector<double> G(xt), S((size_t)nc * nc), w;
+            G.insert(G.end(), at.begin(), at.end());
+            host_gemm(true, false, nc, nc, m, 1.0, G.data(), m, G.data(), m, 0.0, S.data(), nc);
             host_syev(nc, S, w);
-            std::vector<double> Zc;
             int kept = 0;
-            for (int q = nc - 1; q >= 0; --q) {
+            for (int q = nc - 1; q >= 0; --q) {   // the kept columns to the front, scaled
                 if (w[q] <= 1e-12 * w[nc - 1]) continue;
-                std::vector<double> col(nc);
-                for (int i = 0; i < nc; ++i) col[i] = S[i + (size_t)nc * q] / std::sqrt(w[q]);
-                std::vector<double> gz = matmul(G, col, m, nc, 1);
-                Zc.insert(Zc.end(), gz.begin(), gz.end());
                 ++kept;
             }
+            std::vector<double> F((size_t)nc * kept), Zc((size_t)m * kept);
+            for (int q = 0; q < kept; ++q)
+                for (int i = 0; i < nc; ++i)
+                    F[i + (size_t)nc * q] = S[i + (size_t)nc * (nc - 1 - q)] / std::sqrt(w[nc - 1 - q]);
+            host_gemm(false, false, m, kept, nc, 1.0, G.data(), m, F.data(), nc, 0.0, Zc.data(), m);
             DBuf<double> Zd, V2((size_t)n * kept), P2((size_t)n * kept), M2((size_t)n * kept);
             Zd.upload(Zc.data(), Zc.size(), s);
             gemm_nn(c, n, kept, m, 1.0, V.get(), n, Zd.get(), m, 0.0, V2.get(), n);
@@ -1401,30 +1474,32 @@ void davidson_rpa(stda_hip_ctx *c, int k, double tol, std::vector<double> &omega
             STDA_HIP_CHECK(hipMemcpyAsync(P.get(), P2.get(), (size_t)n * kept * 8, hipMemcpyDeviceToDevice, s));
             STDA_HIP_CHECK(hipMemcpyAsync(M.get(), M2.get(), (size_t)n * kept * 8, hipMemcpyDeviceToDevice, s));
             // reduced matrices in the new basis: Zc^T Ap Zc
-            std::vector<double> zt((size_t)kept * m);
-            for (int j = 0; j < kept; ++j)
-                for (int i = 0; i < m; ++i) zt[j + (size_t)kept * i] = Zc[i + (size_t)m * j];
-            std::vector<double> ap2 = matmul(zt, matmul(ap, Zc, m, m, kept), kept, m, kept);
-            std::vector<double> am2 = matmul(zt, matmul(am, Zc, m, m, kept), kept, m, kept);
-            std::fill(Ap.begin(), Ap.end(), 0.0);
-            std::fill(Am.begin(), Am.end(), 0.0);
-            for (int j = 0; j < kept; ++j)
-                for (int i = 0; i < kept; ++i) {
-                    Ap[i + (size_t)maxdim * j] = ap2[i + (size_t)kept * j];
-                    Am[i + (size_t)maxdim * j] = am2[i + (size_t)kept * j];
-                }
+            auto reduce = [&](std::vector<double> &A) {
+                std::vector<double> x((size_t)m * kept), y((size_t)kept * kept);
+                host_gemm(false, false, m, kept, m, 1.0, A.data(), maxdim, Zc.data(), m, 0.0, x.data(), m);
+                host_gemm(true, false, kept, kept, m, 1.0, Zc.data(), m, x.data(), m, 0.0, y.data(), kept);
+                std::fill(A.begin(), A.end(), 0.0);
+                for (int j = 0; j < kept; ++j)
+                    for (int i = 0; i < kept; ++i)
+                        A[i + (size_t)maxdim * j] = 0.5 * (y[i + (size_t)kept * j] + y[j + (size_t)kept * i]);
+            };
+            reduce(Ap);
+            reduce(Am);
             m = kept;
             c->sync();
         }
-        int room = std::min(nun, maxdim - m);
-        STDA_HIP_CHECK(hipMemcpyAsync(V.get() + n * m, R.get(), (size_t)n * room * 8,
-                                      hipMemcpyDeviceToDevice, s));
-        mnew = orthonormalize(c, V.get(), m, V.get() + n * m, room, tmp);
-        // every new direction lies in the space although residuals are above the
-        // tolerance: the iteration cannot progress
-        if (mnew == 0) {
-            if (o.allow_unconverged) return;
-            throw Error(STDA_HIP_ERR_NOT_CONVERGED, "RPA Davidson did not converge (no new directions)");
+        const int room = std::min(nun, maxdim - m);
+        // the first room unconverged residuals, preconditioned, in column order
+        launch_precondition_compact(s, n, 2 * kk, R.get(), c->ed.get(), om, nrm.get(), tol, room,
+                                    V.get() + n * m);
+        if (devortho && room <= 64) {
+            orthonormalize_dev(c, V.get(), m, V.get() + n * m, room, T2.get(), ow.get(),
+                               Hc.get() + (size_t)2 * (m + room) * room);
+            mnew = room;
+            flags_pending = true;
+        } else {
+            mnew = orthonormalize(c, V.get(), m, V.get() + n * m, room, tmp);
+            if (mnew == 0) { no_progress(); return; }
         }
     }
     throw Error(STDA_HIP_ERR_NOT_CONVERGED, "RPA Davidson did not converge");
@@ -2274,10 +2349,14 @@ int stda_hip_solve_tda(stda_hip_ctx *c, int32_t nroots, int32_t capacity, int32_
             int64_t cnt = 0;
             for (double e : c->ed_h) cnt += e <= c->thr;
             int k = (int)std::min<int64_t>(n, cnt + 8);
-            while (true) {
-                davidson_tda(c, k, tol, w, X);
+            DavOpts all;
+            all.window = c->thr;
+            // (once enlarged, the roots at the window's edge are no longer those that
+            // converge first by far: a smaller tolerance makes up for it)
+            for (double t = tol;; t = 0.02 * tol) {
+                davidson_tda(c, k, t, w, X, all);
                 if (w.back() > c->thr || k >= n) break;
-                k = (int)std::min<int64_t>(n, 2 * (int64_t)k);
+                k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));
             }
             int keep = 0;
             for (double e : w) keep += (e > 0.0 && e <= c->thr);
@@ -2356,10 +2435,14 @@ int stda_hip_solve_rpa(stda_hip_ctx *c, int32_t nroots, int32_t capacity, double
             int64_t cnt = 0;
             for (double e : c->ed_h) cnt += e <= c->thr;
             int k = (int)std::min<int64_t>(n, cnt + 8);
-            while (true) {
-                davidson_rpa(c, k, tol, w, XpY, XmY);
+            DavOpts all;
+            all.window = c->thr;
+            // (once enlarged, the roots at the window's edge are no longer those that
+            // converge first by far: a smaller tolerance makes up for it)
+            for (double t = tol;; t = 0.02 * tol) {
+                davidson_rpa(c, k, t, w, XpY, XmY, all);
                 if (w.back() > c->thr || k >= n) break;
-                k = (int)std::min<int64_t>(n, 2 * (int64_t)k);
+                k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));
             }
             int keep = 0;
             for (double e : w) keep += (e * e <= c->thr * c->thr);   // srpapack.f:84-89
@@ -2443,7 +2526,8 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
         // `limit` = its current size instead
         int cap = (int)std::min<int64_t>(maxdim, std::max(2 * need, 128)), limit = maxdim;
         DBuf<double> V((size_t)n * cap), P((size_t)n * cap), M((size_t)n * cap), tmp;
-        DBuf<double> R((size_t)n * 2 * nrhs), XP((size_t)n * nrhs), nrm(2 * nrhs), Yd;
+        DBuf<double> R((size_t)n * 2 * nrhs), XP((size_t)n * nrhs), nrm(2 * nrhs), Yd,
+            VA((size_t)n * nrhs), VB((size_t)n * nrhs);
         // initial space: the right-hand sides preconditioned by the diagonal
         STDA_HIP_CHECK(hipMemcpyAsync(V.get(), rhs.get(), (size_t)n * 3 * 8, hipMemcpyDeviceToDevice, s));
         std::vector<double> zero3(3, 0.0);
@@ -2452,6 +2536,14 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
         launch_precondition(s, n, 3, V.get(), c->ed.get(), z3.get(), V.get());
         int m = 0, mnew = orthonormalize(c, V.get(), 0, V.get(), 3, tmp);
         int m0 = mnew;   // the initial block, kept through restarts
+        // blocks of up to 64 residuals are orthonormalised on the device
+        const bool devortho = 2 * nrhs <= 64;
+        bool flags_pending = false;   // alive flags of the new block still on the device
+        DBuf<double> Hc, T2, ow, alive;
+        if (devortho) {
+            T2.resize((size_t)n * 2 * nrhs);
+            alive.resize(2 * (size_t)nrhs);
+        }
         std::vector<double> rhsnorm(3);
         {
             DBuf<double> rn(3);
@@ -2492,85 +2584,149 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                 limit = cap;
             }
         };
-        for (int it = 0; it < 500 && !done; ++it) {
-            if (mnew > 0) {   // operator images and reduced matrices of the new block
-                apply_ops(c, OP_APB, OP_AMB, mnew, V.get() + n * m, n, P.get() + n * m, n,
-                          M.get() + n * m, n, fp32);
-                const int mt = m + mnew;
-                DBuf<double> Hc((size_t)mt * mnew * 2 + (size_t)mnew * 3);
-                dgemm_tn(c, mt, mnew, n, V.get(), n, P.get() + n * m, n, Hc.get());
-                dgemm_tn(c, mt, mnew, n, V.get(), n, M.get() + n * m, n, Hc.get() + (size_t)mt * mnew);
-                dgemm_tn(c, mnew, 3, n, V.get() + n * m, n, rhs.get(), n, Hc.get() + (size_t)2 * mt * mnew);
-                std::vector<double> hc((size_t)mt * mnew * 2 + (size_t)mnew * 3);
-                Hc.download(hc.data(), hc.size(), s);
-                c->sync();
-                for (int j = 0; j < mnew; ++j)
-                    for (int i = 0; i < mt; ++i) {
-                        double vp = hc[i + (size_t)mt * j], vm = hc[(size_t)mt * mnew + i + (size_t)mt * j];
-                        Ap[i + (size_t)maxdim * (m + j)] = vp; Ap[(m + j) + (size_t)maxdim * i] = vp;
-                        Am[i + (size_t)maxdim * (m + j)] = vm; Am[(m + j) + (size_t)maxdim * i] = vm;
-                    }
-                for (int r = 0; r < 3; ++r)
-                    for (int j = 0; j < mnew; ++j) Br[(m + j) + (size_t)maxdim * r] = hc[(size_t)2 * mt * mnew + j + (size_t)mnew * r];
-                m = mt;
-            }
-            // Reduced problem, one factorisation for every frequency: with
-            // Am = L L^T and L^T Ap L = Z diag(lam) Z^T (lam: the space's RPA
-            // w_n^2), (Ap - w^2 Am^-1) a = V^T r gives a = L Z c with
-            // c = (lam - w^2)^-1 Z^T L^T V^T r, and b = w Am^-1 a = w L^-T Z c.
-            std::vector<double> ap((size_t)m * m), am((size_t)m * m);
-            for (int j = 0; j < m; ++j)
-                for (int i = 0; i < m; ++i) {
-                    ap[i + (size_t)m * j] = 0.5 * (Ap[i + (size_t)maxdim * j] + Ap[j + (size_t)maxdim * i]);
-                    am[i + (size_t)m * j] = 0.5 * (Am[i + (size_t)maxdim * j] + Am[j + (size_t)maxdim * i]);
-                }
-            std::vector<double> L(am);
-            if (!host_potrf_lower(m, L)) throw Error(STDA_HIP_ERR_AMB_NOT_PD, "A-B not positive definite");
-            std::vector<double> t1((size_t)m * m), Z((size_t)m * m), lam;
-            host_gemm(false, false, m, m, m, 1.0, ap.data(), m, L.data(), m, 0.0, t1.data(), m);
-            host_gemm(true, false, m, m, m, 1.0, L.data(), m, t1.data(), m, 0.0, Z.data(), m);
+        std::vector<double> ap, L, inv, t1, W, Yz, lam;
+        bool spectral = false;      // W, Yz and lam are those of the current space
+        // The space's RPA pairs: with Am = L L^T and L^T Ap L = Z diag(lam) Z^T
+        // (lam: the space's w_n^2), W = L Z, Yz = L^-T Z; then a = W c and
+        // b = w Yz c with c = (lam - w^2)^-1 W^T V^T r.
+        auto spectrum = [&]() {
+            if (spectral) return;
+            std::vector<double> t((size_t)m * m), Z((size_t)m * m);
+            host_gemm(false, false, m, m, m, 1.0, ap.data(), m, L.data(), m, 0.0, t.data(), m);
+            host_gemm(true, false, m, m, m, 1.0, L.data(), m, t.data(), m, 0.0, Z.data(), m);
             for (int j = 0; j < m; ++j)
                 for (int i = 0; i < j; ++i) {
                     double v = 0.5 * (Z[i + (size_t)m * j] + Z[j + (size_t)m * i]);
                     Z[i + (size_t)m * j] = v; Z[j + (size_t)m * i] = v;
                 }
             host_syev(m, Z, lam);
-            std::vector<double> W((size_t)m * m), Yz(Z), G((size_t)m * 3);
+            W.assign((size_t)m * m, 0.0);
             host_gemm(false, false, m, m, m, 1.0, L.data(), m, Z.data(), m, 0.0, W.data(), m);
+            Yz.swap(Z);
             host_solve_lt(m, m, L, Yz.data(), m);
-            host_gemm(true, false, m, 3, m, 1.0, W.data(), m, Br.data(), maxdim, 0.0, G.data(), m);
-            const double lamscale = std::max(1.0, std::fabs(lam[m - 1]));
-            coef.assign((size_t)m * 2 * nrhs, 0.0);
-            std::vector<double> cv((size_t)m * 3);
-            for (int f = 0; f < nfreq; ++f) {
-                const double w = omega[f];
-                for (int r = 0; r < 3; ++r)
-                    for (int q = 0; q < m; ++q) {
-                        double den = lam[q] - w * w;
-                        if (std::fabs(den) < 1.0e-300 * lamscale) den = den < 0.0 ? -1.0e-300 : 1.0e-300;
-                        cv[q + (size_t)m * r] = G[q + (size_t)m * r] / den;
+            spectral = true;
+        };
+        for (int it = 0; it < 500 && !done; ++it) {
+            if (mnew > 0) {   // operator images and reduced matrices of the new block
+                apply_ops(c, OP_APB, OP_AMB, mnew, V.get() + n * m, n, P.get() + n * m, n,
+                          M.get() + n * m, n, fp32);
+                const int mt = m + mnew;
+                const size_t blk = (size_t)mt * mnew, nh = 2 * blk + (size_t)mnew * 3;
+                // [V^T P | V^T M | V^T r] of the new columns, and their alive flags
+                Hc.ensure(nh + mnew);
+                dgemm_tn(c, mt, mnew, n, V.get(), n, P.get() + n * m, n, Hc.get());
+                dgemm_tn(c, mt, mnew, n, V.get(), n, M.get() + n * m, n, Hc.get() + blk);
+                dgemm_tn(c, mnew, 3, n, V.get() + n * m, n, rhs.get(), n, Hc.get() + 2 * blk);
+                double *hc = c->pinned(nh + mnew);
+                STDA_HIP_CHECK(hipMemcpyAsync(hc, Hc.get(), nh * 8, hipMemcpyDeviceToHost, s));
+                if (flags_pending)
+                    STDA_HIP_CHECK(hipMemcpyAsync(hc + nh, alive.get(), (size_t)mnew * 8,
+                                                  hipMemcpyDeviceToHost, s));
+                c->sync();
+                // columns that brought nothing (zero) leave the space
+                std::vector<int> keep;
+                for (int j = 0; j < mnew; ++j)
+                    if (!flags_pending || hc[nh + j] != 0.0) keep.push_back(j);
+                flags_pending = false;
+                const int nk = (int)keep.size();
+                // Every new direction already lies in the space although the
+                // residuals are above the tolerance: the iteration cannot progress.
+                if (nk == 0)
+                    throw Error(STDA_HIP_ERR_NOT_CONVERGED,
+                                "response solver did not converge (no new directions)");
+                for (int j = 0; j < nk; ++j) {
+                    const int cj = keep[j];
+                    if (cj != j)
+                        for (DBuf<double> *B : {&V, &P, &M})
+                            STDA_HIP_CHECK(hipMemcpyAsync(B->get() + n * (m + j), B->get() + n * (m + cj),
+                                                          (size_t)n * 8, hipMemcpyDeviceToDevice, s));
+                    for (int i = 0; i < m + nk; ++i) {
+                        const int ci = i < m ? i : m + keep[i - m];
+                        const double vp = hc[ci + (size_t)mt * cj], vm = hc[blk + ci + (size_t)mt * cj];
+                        Ap[i + (size_t)maxdim * (m + j)] = vp; Ap[(m + j) + (size_t)maxdim * i] = vp;
+                        Am[i + (size_t)maxdim * (m + j)] = vm; Am[(m + j) + (size_t)maxdim * i] = vm;
                     }
-                host_gemm(false, false, m, 3, m, 1.0, W.data(), m, cv.data(), m, 0.0,
-                          coef.data() + (size_t)m * 3 * f, m);
-                host_gemm(false, false, m, 3, m, w, Yz.data(), m, cv.data(), m, 0.0,
-                          coef.data() + (size_t)m * (nrhs + 3 * f), m);
+                    for (int r = 0; r < 3; ++r)
+                        Br[(m + j) + (size_t)maxdim * r] = hc[2 * blk + cj + (size_t)mnew * r];
+                }
+                m += nk;
+            }
+            // Reduced problem (Ap - w^2 Am^-1) a = V^T r, b = w Am^-1 a for every
+            // frequency: the inverse of the positive definite Am once, then a
+            // Cholesky (above a pole: symmetric indefinite) solve per frequency.  One eigenproblem for all
+            // of them (below) takes several times as long from 100 vectors on, and
+            // serves the restarts and a breakdown.
+            ap.resize((size_t)m * m);
+            L.resize((size_t)m * m);
+            for (int j = 0; j < m; ++j)
+                for (int i = 0; i < m; ++i) {
+                    ap[i + (size_t)m * j] = 0.5 * (Ap[i + (size_t)maxdim * j] + Ap[j + (size_t)maxdim * i]);
+                    L[i + (size_t)m * j] = 0.5 * (Am[i + (size_t)maxdim * j] + Am[j + (size_t)maxdim * i]);
+                }
+            if (!host_potrf_lower(m, L)) throw Error(STDA_HIP_ERR_AMB_NOT_PD, "A-B not positive definite");
+            coef.assign((size_t)m * 2 * nrhs, 0.0);
+            spectral = false;
+            bool solved = true;
+            if (wmax > 0.0) {
+                inv = L;
+                solved = host_potri(m, inv);
+            }
+            for (int f = 0; solved && f < nfreq; ++f) {
+                const double w = omega[f];
+                auto shifted = [&]() {
+                    t1 = ap;
+                    if (w != 0.0)
+                        for (size_t q = 0; q < t1.size(); ++q) t1[q] -= w * w * inv[q];
+                };
+                double *xa = coef.data() + (size_t)m * 3 * f, *xb = coef.data() + (size_t)m * (nrhs + 3 * f);
+                for (int r = 0; r < 3; ++r)
+                    std::copy(Br.begin() + (size_t)maxdim * r, Br.begin() + (size_t)maxdim * r + m,
+                              xa + (size_t)m * r);
+                shifted();   // positive definite below the space's first pole
+                solved = host_potrf_lower(m, t1) && host_potrs(m, 3, t1, xa, m);
+                if (!solved) {
+                    shifted();
+                    solved = host_sysv(m, 3, t1, xa, m);
+                }
+                if (solved && w != 0.0)
+                    host_gemm(false, false, m, 3, m, w, inv.data(), m, xa, m, 0.0, xb, m);
+            }
+            if (!solved) {
+                spectrum();
+                std::vector<double> cv((size_t)m * 3), G((size_t)m * 3);
+                host_gemm(true, false, m, 3, m, 1.0, W.data(), m, Br.data(), maxdim, 0.0, G.data(), m);
+                const double lamscale = std::max(1.0, std::fabs(lam[m - 1]));
+                for (int f = 0; f < nfreq; ++f) {
+                    const double w = omega[f];
+                    for (int r = 0; r < 3; ++r)
+                        for (int q = 0; q < m; ++q) {
+                            double den = lam[q] - w * w;
+                            if (std::fabs(den) < 1.0e-300 * lamscale) den = den < 0.0 ? -1.0e-300 : 1.0e-300;
+                            cv[q + (size_t)m * r] = G[q + (size_t)m * r] / den;
+                        }
+                    host_gemm(false, false, m, 3, m, 1.0, W.data(), m, cv.data(), m, 0.0,
+                              coef.data() + (size_t)m * 3 * f, m);
+                    host_gemm(false, false, m, 3, m, w, Yz.data(), m, cv.data(), m, 0.0,
+                              coef.data() + (size_t)m * (nrhs + 3 * f), m);
+                }
             }
             // residuals R1 = P a - w V b - r ; R2 = M b - w V a
-            Yd.upload(coef.data(), coef.size(), s);
-            DBuf<double> VB((size_t)n * nrhs), VA((size_t)n * nrhs);
-            gemm_nn(c, n, nrhs, m, 1.0, P.get(), n, Yd.get(), m, 0.0, R.get(), n);
-            gemm_nn(c, n, nrhs, m, 1.0, V.get(), n, Yd.get() + (size_t)m * nrhs, m, 0.0, VB.get(), n);
-            gemm_nn(c, n, nrhs, m, 1.0, V.get(), n, Yd.get(), m, 0.0, VA.get(), n);
-            gemm_nn(c, n, nrhs, m, 1.0, M.get(), n, Yd.get() + (size_t)m * nrhs, m, 0.0,
-                    R.get() + n * nrhs, n);
+            double *pin = c->pinned(coef.size() + 2 * (size_t)nrhs);
+            std::copy(coef.begin(), coef.end(), pin);
+            Yd.resize(coef.size());
+            STDA_HIP_CHECK(hipMemcpyAsync(Yd.get(), pin, coef.size() * 8, hipMemcpyHostToDevice, s));
+            const double *ya = Yd.get(), *yb = ya + (size_t)m * nrhs;
+            gemm_nn2(c, n, nrhs, m, P.get(), V.get(), n, ya, m, R.get(), VA.get(), n);
+            gemm_nn2(c, n, nrhs, m, M.get(), V.get(), n, yb, m, R.get() + n * nrhs, VB.get(), n);
             launch_residual(s, n, nrhs, R.get(), VB.get(), wd.get(), R.get());
-            launch_residual(s, n, nrhs, R.get() + n * nrhs, VA.get(), wd.get(), R.get() + n * nrhs);
             for (int f = 0; f < nfreq; ++f)   // subtract the right-hand sides: R1 -= r
                 launch_residual(s, n, 3, R.get() + n * 3 * f, rhs.get(), oned.get(),
                                 R.get() + n * 3 * f);
-            col_norms(c, n, 2 * nrhs, R.get(), nrm.get());
-            std::vector<double> rn(2 * nrhs);
-            nrm.download(rn.data(), rn.size(), s);
+            residual_norms(c, n, nrhs, R.get() + n * nrhs, VA.get(), wd.get(), R.get() + n * nrhs,
+                           nrm.get() + nrhs);
+            col_norms(c, n, nrhs, R.get(), nrm.get());
+            double *rn = pin + coef.size();
+            STDA_HIP_CHECK(hipMemcpyAsync(rn, nrm.get(), 2 * (size_t)nrhs * 8, hipMemcpyDeviceToHost, s));
             c->sync();
             std::vector<int> un;
             const double tol_now = fp32 ? tol32 : tol;
@@ -2649,6 +2805,7 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                     e[i] = 0.0;
                 }
                 for (int col = 0; col < 2 * nrhs; ++col) add_col(coef.data() + (size_t)m * col);
+                spectrum();
                 const int room = std::max(0, (limit / 2 - m0 - 2 * nrhs) / 2);
                 for (int q = 0, added = 0; q < m && added < room && wmax > 0.0; ++q) {
                     if (!(lam[q] > 0.0) || lam[q] > 1.5625 * wmax * wmax) break;
@@ -2664,15 +2821,15 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                     STDA_HIP_CHECK(hipMemcpyAsync(B->get(), rs.get(), (size_t)n * r * 8,
                                                   hipMemcpyDeviceToDevice, s));
                 }
-                auto reduce = [&](const std::vector<double> &a, std::vector<double> &out) {
+                auto reduce = [&](std::vector<double> &out) {
                     std::vector<double> aq((size_t)m * r), qaq((size_t)r * r);
-                    host_gemm(false, false, m, r, m, 1.0, a.data(), m, Q.data(), m, 0.0, aq.data(), m);
+                    host_gemm(false, false, m, r, m, 1.0, out.data(), maxdim, Q.data(), m, 0.0, aq.data(), m);
                     host_gemm(true, false, r, r, m, 1.0, Q.data(), m, aq.data(), m, 0.0, qaq.data(), r);
                     for (int j = 0; j < r; ++j)
                         for (int i = 0; i < r; ++i) out[i + (size_t)maxdim * j] = qaq[i + (size_t)r * j];
                 };
-                reduce(ap, Ap);
-                reduce(am, Am);
+                reduce(Ap);
+                reduce(Am);
                 std::vector<double> br((size_t)maxdim * 3, 0.0);
                 host_gemm(true, false, r, 3, m, 1.0, Q.data(), m, Br.data(), maxdim, 0.0, br.data(), maxdim);
                 Br.swap(br);
@@ -2682,12 +2839,19 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
             }
             if (nun <= 0) throw Error(STDA_HIP_ERR_NOT_CONVERGED, "response subspace exhausted");
             STDA_HIP_CHECK(hipMemcpyAsync(V.get() + n * m, R.get(), (size_t)n * nun * 8, hipMemcpyDeviceToDevice, s));
-            mnew = orthonormalize(c, V.get(), m, V.get() + n * m, nun, tmp);
-            // Every new direction already lies in the space although the
-            // residuals are above the tolerance: the iteration cannot progress.
-            if (mnew == 0)
-                throw Error(STDA_HIP_ERR_NOT_CONVERGED,
-                            "response solver did not converge (no new directions)");
+            if (devortho) {
+                ow.ensure(3 * (size_t)(m + nun) * nun + (size_t)nun * nun + 1);
+                orthonormalize_dev(c, V.get(), m, V.get() + n * m, nun, T2.get(), ow.get(), alive.get());
+                mnew = nun;
+                flags_pending = true;
+            } else {
+                mnew = orthonormalize(c, V.get(), m, V.get() + n * m, nun, tmp);
+                // Every new direction already lies in the space although the
+                // residuals are above the tolerance: the iteration cannot progress.
+                if (mnew == 0)
+                    throw Error(STDA_HIP_ERR_NOT_CONVERGED,
+                                "response solver did not converge (no new directions)");
+            }
         }
         if (!done) throw Error(STDA_HIP_ERR_NOT_CONVERGED, "response solver did not converge");
         // alpha_rc = -2 mu_r^T (X+Y)_c (linear_response.f:147-172)
