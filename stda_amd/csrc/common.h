@@ -186,6 +186,12 @@ void launch_mu_blocks(hipStream_t s, const double *moments, int64_t npk, int no,
 // direction the integral kernel's recurrence tables are sized for (checked on the host).
 constexpr int AO_LMAX = 4;
 void launch_pack_upper(hipStream_t s, int64_t n, const double *P, double *out);
+// S^1/2 by coupled Newton-Schulz steps: Y = (1.8 / bound) S, Z = I with bound
+// (zeroed before) the largest row sum of |S| as the bits of a double; and
+// W <- (3 I - W) / 2 with the largest |W - I| in dev (zeroed before)
+void launch_root_init(hipStream_t s, int n, const double *S, unsigned long long *bound, double *Y,
+                      double *Z);
+void launch_root_step(hipStream_t s, int n, double *W, unsigned long long *dev);
 void launch_scale_rows(hipStream_t s, int64_t m, int64_t k, const double *f, double *T);
 void launch_ao_ints(hipStream_t s, int nao, const int64_t *ptr, const double *alpha,
                     const double *coef, const double *cen, const int32_t *lmn, double *S,

@@ -1,12 +1,14 @@
 // Device parts of the upstream transforms (the AO -> MO moments of onetri and
 // shrink, stda.f:351-412 and 1695-1706, and the Loewdin orthogonalisation of
-// makel, stda.f:430-452 and 1615-1691): the products themselves are rocBLAS
-// GEMMs and a rocSOLVER eigensolve on the host side; these kernels pack and
+// makel, stda.f:430-452 and 1615-1691): the products themselves, among them
+// the iteration for S^1/2, are the matrix-core GEMM's; these kernels pack and
 // scale (HBM-bound element-wise passes), and compute the one-electron AO
 // integrals the transforms start from (libcint.f:252-352, 653-756;
 // intpack.f90:1208-1283), one thread per AO pair.
 
 #include "common.h"
+
+#include <algorithm>
 
 // the integrals keep the operation order of the host recurrences (no contraction)
 #pragma clang fp contract(off)
@@ -114,7 +116,68 @@ unsigned grid_for(int64_t n) {
     return (unsigned)(b < 8192 ? (b > 0 ? b : 1) : 8192);
 }
 
+// Largest absolute row sum of the symmetric matrix whose upper triangle S holds
+// (an upper bound of its eigenvalues), as the bits of a non-negative double
+__global__ void __launch_bounds__(256) row_bound_kernel(int n, const double *__restrict__ S,
+                                                        unsigned long long *bound) {
+    __shared__ double ws[4];
+    const int i = blockIdx.x;
+    double a = 0.0;
+    for (int j = threadIdx.x; j < n; j += 256)
+        a += fabs(i <= j ? S[i + (int64_t)n * j] : S[j + (int64_t)n * i]);
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = a;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(bound, (unsigned long long)__double_as_longlong(ws[0] + ws[1] + ws[2] + ws[3]));
+}
+
+// Y = (1.8 / bound) S (both triangles from the upper one), Z = I
+__global__ void root_init_kernel(int n, const double *__restrict__ S,
+                                 const unsigned long long *__restrict__ bound, double *Y, double *Z) {
+    const double f = 1.8 / __longlong_as_double((long long)*bound);
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < (int64_t)n * n;
+         e += (int64_t)gridDim.x * blockDim.x) {
+        const int i = (int)(e % n), j = (int)(e / n);
+        Y[e] = f * (i <= j ? S[e] : S[j + (int64_t)n * i]);
+        Z[e] = i == j ? 1.0 : 0.0;
+    }
+}
+
+// W <- 1.5 I - 0.5 W, and the largest |W - I| into dev (bits; NaN counts as infinite)
+__global__ void __launch_bounds__(256) root_step_kernel(int n, double *W, unsigned long long *dev) {
+    __shared__ double ws[4];
+    double d = 0.0;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < (int64_t)n * n;
+         e += (int64_t)gridDim.x * blockDim.x) {
+        const double one = e % n == e / n ? 1.0 : 0.0, w = W[e];
+        const double x = fabs(w - one);
+        d = x <= 1.0e300 ? fmax(d, x) : 1.0e300;
+        W[e] = 1.5 * one - 0.5 * w;
+    }
+    for (int o = 32; o > 0; o >>= 1) d = fmax(d, __shfl_xor(d, o, 64));
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = d;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(dev, (unsigned long long)__double_as_longlong(
+                           fmax(fmax(ws[0], ws[1]), fmax(ws[2], ws[3]))));
+}
+
 }  // namespace
+
+void launch_root_init(hipStream_t s, int n, const double *S, unsigned long long *bound, double *Y,
+                      double *Z) {
+    hipLaunchKernelGGL(row_bound_kernel, dim3(n), dim3(256), 0, s, n, S, bound);
+    hipLaunchKernelGGL(root_init_kernel, dim3(grid_for((int64_t)n * n)), dim3(256), 0, s, n, S,
+                       bound, Y, Z);
+    STDA_HIP_CHECK(hipGetLastError());
+}
+
+void launch_root_step(hipStream_t s, int n, double *W, unsigned long long *dev) {
+    hipLaunchKernelGGL(root_step_kernel, dim3(std::min(grid_for((int64_t)n * n), 512u)), dim3(256), 0,
+                       s, n, W, dev);
+    STDA_HIP_CHECK(hipGetLastError());
+}
 
 void launch_pack_upper(hipStream_t s, int64_t n, const double *P, double *out) {
     if (n <= 0) return;
