@@ -2101,6 +2101,17 @@ static void tda_properties(stda_hip_ctx *c, const double *X, const std::vector<d
     tda_props_from_moments(c->ak, w, T.data(), T2.empty() ? nullptr : T2.data(), props, alpha);
 }
 
+// Whether a mixed-precision solve uses the FP32 operator: from 4e8 flops per vector
+// and product on (about 165 atoms in a minimal basis).  Below, an iteration is
+// launches and the subspace step, the product's precision hardly shows in its
+// time (133 atoms, 20 vectors: 0.19 ms in FP64, 0.12 in FP32, of 0.6), and FP64
+// throughout to the refinement's tolerance needs three iterations fewer.
+static bool fp32_operator(const stda_hip_ctx *c) {
+    const double per = 4.0 * c->nao * (double)c->no * (c->nv + (double)c->nao);
+    return c->precision == 2 || (c->precision == 1 && per >= 4.0e8);
+}
+constexpr double kMixedTol = 1.0e-7;   // residual tolerance of a mixed-precision solve's FP64 end
+
 // Mixed precision TDA: FP32 operator to a residual of max(tol, 1e-6), then up to
 // four FP64 iterations: Rayleigh-Ritz in the span of the converged vectors, and
 // three with preconditioned residuals added, or to max(tol, 1e-7).  (The first
@@ -2112,6 +2123,10 @@ static void tda_properties(stda_hip_ctx *c, const double *X, const std::vector<d
 // noise floor) and the FP32 phase starts from its Ritz vectors.
 static void solve_tda_mixed(stda_hip_ctx *c, int nroots, double tol, std::vector<double> &w,
                             DBuf<double> &X) {
+    if (!fp32_operator(c)) {
+        davidson_tda(c, nroots, std::max(tol, kMixedTol), w, X);
+        return;
+    }
     DavOpts lo;
     lo.fp32 = true;
     if (c->precision == 2) {
@@ -2134,7 +2149,7 @@ static void solve_tda_mixed(stda_hip_ctx *c, int nroots, double tol, std::vector
     ref.allow_unconverged = true;
     DBuf<double> X0 = std::move(X);
     HostSpan hs(c, "mixed_fp64_refine");
-    davidson_tda(c, nroots, std::max(tol, 1.0e-7), w, X, ref);
+    davidson_tda(c, nroots, std::max(tol, kMixedTol), w, X, ref);
 }
 
 static void rpa_properties(stda_hip_ctx *c, const double *XpY, const double *XmY,
@@ -2397,7 +2412,9 @@ int stda_hip_solve_rpa(stda_hip_ctx *c, int32_t nroots, int32_t capacity, double
         std::vector<double> w;
         DBuf<double> XpY, XmY;
         const int64_t n = c->nci;
-        if (nroots > 0 && c->precision >= 1) {
+        if (nroots > 0 && c->precision >= 1 && !fp32_operator(c)) {
+            davidson_rpa(c, nroots, std::max(tol, kMixedTol), w, XpY, XmY);
+        } else if (nroots > 0 && c->precision >= 1) {
             DavOpts lo;
             lo.fp32 = true;
             DBuf<double> Vb;
@@ -2486,8 +2503,8 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
         // any useful tolerance.  The iteration runs with the FP32 operator until
         // its residuals reach max(tol, 1e-6) or stop falling, then the space's
         // operator images are recomputed in FP64 and it finishes in FP64.
-        bool fp32 = c->precision >= 1;
-        if (fp32) tol = std::max(tol, 1.0e-8);
+        bool fp32 = fp32_operator(c);
+        if (c->precision >= 1) tol = std::max(tol, 1.0e-8);
         c->gemm32 = c->precision == 2 ? GEMM_BF16X3 : GEMM_F32;
         const double tol32 = std::max(tol, c->precision == 2 ? 3.0e-5 : 1.0e-6);
         double best32 = 1.0e300;
