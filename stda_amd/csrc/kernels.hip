@@ -715,7 +715,6 @@ namespace stda {
 typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int M_T = 8;          // per-dimension tile size
 constexpr int M_CH = 16;        // atoms per staged chunk (4 MFMA k-steps)
-constexpr int M_LD = 64 + 1;    // padded LDS row (doubles)
 
 }  // namespace stda
 
@@ -769,13 +768,18 @@ namespace stda {
 // (tile, atom chunk) steps are flattened; while the matrix cores work on step
 // s from one LDS buffer, the operands of step s+1 are fetched into registers
 // and then written to the other buffer, so a single barrier per step orders
-// everything.
+// everything.  The matrix cores bound it (59 % busy at 180 atoms in a split-valence
+// basis before the addresses were kept and the LDS conflicts went, 41 TFLOP/s of
+// couplings; 115 -> 102 ms there, 5.28 -> 4.79 ms at 200 atoms in a minimal basis).
+// LDS rows of 68 elements: in FP64 the two rows that half a wave reads then fall
+// into distinct banks (65 left every read with conflicts, 17 % of the LDS time),
+// and rows 8.. shift by 4 more so that the writes do too.
+constexpr int PIPE_LD = 68;
+__device__ __forceinline__ constexpr int pipe_row(int row) { return row * PIPE_LD + (row >> 3) * 4; }
 template <typename T, int CH>
 struct PipeBuf {
-    T pk[CH][M_LD];
-    T qc[CH][M_LD];
-    T pj[CH][M_LD];
-    T qv[CH][M_LD];
+    static constexpr int N = CH * PIPE_LD + (CH / 8) * 4;
+    T pk[N], qc[N], pj[N], qv[N];
 };
 template <typename T, int CH>
 struct PipeSmem {
@@ -801,25 +805,6 @@ template <> struct PipeMfma<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
 };
-
-// Column index (pair or packed pair) of this thread's VPT staged vectors of
-// each operand (vectors vb + VS r), or -1.  o = 0 pK(k,c), 1 q(j,b),
-// 2 pJ(k,j), 3 qab(c,b); the row tile gives k, c and the column tile j, b.
-template <int VS, int VPT>
-__device__ __forceinline__ void stage_cols(TileSet rows, int rt, TileSet cols, int ct, int nv,
-                                           int vb, int32_t idx[4][VPT]) {
-#pragma unroll
-    for (int r = 0; r < VPT; ++r) {
-        int v = vb + VS * r, x = v / M_T, y = v % M_T;
-        int kx = rows.occ[rt * M_T + x], cy = rows.vir[rt * M_T + y];
-        int jx = cols.occ[ct * M_T + x], by = cols.vir[ct * M_T + y];
-        int jy = cols.occ[ct * M_T + y], cx = rows.vir[rt * M_T + x];
-        idx[0][r] = (kx >= 0 && cy >= 0) ? kx * nv + cy : -1;
-        idx[1][r] = (jx >= 0 && by >= 0) ? jx * nv + by : -1;
-        idx[2][r] = (kx >= 0 && jy >= 0) ? (int32_t)lin0(kx, jy) : -1;
-        idx[3][r] = (cx >= 0 && by >= 0) ? (int32_t)lin0(cx, by) : -1;
-    }
-}
 
 // de of a row pair (k,c) or column pair (j,b) of a tile; NaN when the pair is
 // outside the tile or not selected by the mask.
@@ -877,7 +862,6 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
     const int ct0 = (int)((int64_t)cols.ntiles * sp / nsplit);
     const int ct1 = (int)((int64_t)cols.ntiles * (sp + 1) / nsplit);
     const int nch = (ncent + CH - 1) / CH;
-    const int64_t nsteps = (int64_t)(ct1 - ct0) * nch;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int kh = w >> 1, jh = w & 1;
     const int r16 = lane & 15, g = lane >> 4, hi = r16 >> 2, lo = r16 & 3;
@@ -899,18 +883,29 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
         for (int i = 0; i < 4; ++i)
             dr[chv][i] = drow[(int64_t)own * PT2_SLOTS + (4 * kh + kk_of(i)) * M_T + 4 * chv + cc_of(i)];
 
-    int32_t idx[4][VPT];
+    // The staged vectors' addresses are kept through a column tile; a vector that
+    // does not exist (an orbital beyond the range) reads the first one, as every
+    // slot that it enters is masked by the NaN of its de.  Only the last chunk of
+    // atoms needs a mask.  (Formed anew for each chunk, addresses and masks and the
+    // division of the step count were four fifths of the vector instructions.)
+    const T *ptr[4][VPT];
     LoadT pre[4][VPT];
-    auto fetch = [&](int ch) {
-        const int a = ch * CH + W * sa;
-        const bool in = a < ncent;
+    auto fetch = [&](int chunk) {
+        const int a0 = chunk * CH;
+        if (a0 + CH <= ncent) {
 #pragma unroll
-        for (int o = 0; o < 4; ++o)
+            for (int o = 0; o < 4; ++o)
 #pragma unroll
-            for (int r = 0; r < VPT; ++r)
-                pre[o][r] = (in && idx[o][r] >= 0)
-                                ? *reinterpret_cast<const LoadT *>(src[o] + lda * idx[o][r] + a)
-                                : LoadT(0);
+                for (int r = 0; r < VPT; ++r)
+                    pre[o][r] = *reinterpret_cast<const LoadT *>(ptr[o][r] + a0);
+        } else {
+            const bool in = a0 + W * sa < ncent;
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+#pragma unroll
+                for (int r = 0; r < VPT; ++r)
+                    pre[o][r] = in ? *reinterpret_cast<const LoadT *>(ptr[o][r] + a0) : LoadT(0);
+        }
     };
     auto store = [&](int b) {
 #pragma unroll
@@ -921,21 +916,56 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
                 T x[4];
 #pragma unroll
                 for (int o = 0; o < 4; ++o) x[o] = pre[o][r][u];
-                sm.buf[b].pk[W * sa + u][v] = x[0];
-                sm.buf[b].qc[W * sa + u][v] = x[1];
-                sm.buf[b].pj[W * sa + u][v] = x[2];
-                sm.buf[b].qv[W * sa + u][v] = x[3];
+                const int e = pipe_row(W * sa + u) + v;
+                sm.buf[b].pk[e] = x[0];
+                sm.buf[b].qc[e] = x[1];
+                sm.buf[b].pj[e] = x[2];
+                sm.buf[b].qv[e] = x[3];
             }
         }
     };
+    // Column (pair or packed pair) of this thread's VPT staged vectors of each
+    // operand (vectors svb + VS r).  o = 0 pK(k,c), 1 q(j,b),
+    // 2 pJ(k,j), 3 qab(c,b); the row tile gives k, c and the column tile j, b.
+    // The row tile's orbitals are read once and a column tile's one tile ahead,
+    // off the path to its first operands.
+    int32_t rk[VPT], rc[VPT], rx[VPT], cj[VPT], cb[VPT], cy[VPT];
+    auto read_cols = [&](int ct) {
+        const int c = min(ct, ct1 - 1);
+#pragma unroll
+        for (int r = 0; r < VPT; ++r) {
+            const int v = svb + VS * r, x = v / M_T, y = v % M_T;
+            cj[r] = cols.occ[c * M_T + x];
+            cb[r] = cols.vir[c * M_T + y];
+            cy[r] = cols.occ[c * M_T + y];
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < VPT; ++r) {
+        const int v = svb + VS * r, x = v / M_T, y = v % M_T;
+        rk[r] = rows.occ[own * M_T + x];
+        rc[r] = rows.vir[own * M_T + y];
+        rx[r] = rows.vir[own * M_T + x];
+    }
     auto set_tile = [&](int other) {
-        stage_cols<VS, VPT>(rows, own, cols, other, nv, svb, idx);
+#pragma unroll
+        for (int r = 0; r < VPT; ++r) {
+            int64_t i[4];
+            i[0] = (rk[r] >= 0 && rc[r] >= 0) ? rk[r] * nv + rc[r] : 0;
+            i[1] = (cj[r] >= 0 && cb[r] >= 0) ? cj[r] * nv + cb[r] : 0;
+            i[2] = (rk[r] >= 0 && cy[r] >= 0) ? lin0(rk[r], cy[r]) : 0;
+            i[3] = (rx[r] >= 0 && cb[r] >= 0) ? lin0(rx[r], cb[r]) : 0;
+#pragma unroll
+            for (int o = 0; o < 4; ++o) ptr[o][r] = src[o] + lda * i[o] + W * sa;
+        }
+        read_cols(other + 1);
 #pragma unroll
         for (int bh = 0; bh < 2; ++bh)
             dcn[bh] = dcol[(int64_t)other * PT2_SLOTS + (4 * jh + hi) * M_T + 4 * bh + lo];
     };
 
-    if (nsteps > 0) {
+    if (ct1 > ct0) {
+        read_cols(ct0);
         set_tile(ct0);
         fetch(0);
         store(0);
@@ -953,33 +983,31 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
     // partial row sums of register i's rows of half chv, index 4 chv + i
     double part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 
-    for (int64_t step = 0; step < nsteps; ++step) {
-        const int ch = (int)(step % nch);
-        const int other = ct0 + (int)(step / nch);
-        const int cur = (int)(step & 1);
-        const bool more = step + 1 < nsteps;
+    int ch = 0, other = ct0, cur = 0;   // atom chunk, column tile, LDS buffer
+    while (other < ct1) {
+        const bool last = ch == nch - 1;
+        const bool more = !last || other + 1 < ct1;
         if (more) {
-            int ch2 = (int)((step + 1) % nch);
-            if (ch2 == 0) set_tile(other + 1);
-            fetch(ch2);
+            if (last) set_tile(other + 1);
+            fetch(last ? 0 : ch + 1);
         }
         const PipeBuf<T, CH> &B = sm.buf[cur];
 #pragma unroll
         for (int s4 = 0; s4 < CH / 4; ++s4) {
-            int arow = 4 * s4 + g;
-            T aJ = B.pj[arow][iPJ];
-            T aK0 = B.pk[arow][iPK0], aK1 = B.pk[arow][iPK0 + 4];
-            T bQ0 = B.qc[arow][iQ0], bQ1 = B.qc[arow][iQ0 + 4];
-            accJ[0] = PipeMfma<T>::step(aJ, B.qv[arow][iQV0], accJ[0]);
-            accJ[1] = PipeMfma<T>::step(aJ, B.qv[arow][iQV0 + 4], accJ[1]);
-            accJ[2] = PipeMfma<T>::step(aJ, B.qv[arow][iQV0 + 32], accJ[2]);
-            accJ[3] = PipeMfma<T>::step(aJ, B.qv[arow][iQV0 + 36], accJ[3]);
+            const int e = pipe_row(4 * s4) + PIPE_LD * g;   // row 4 s4 + g
+            T aJ = B.pj[e + iPJ];
+            T aK0 = B.pk[e + iPK0], aK1 = B.pk[e + iPK0 + 4];
+            T bQ0 = B.qc[e + iQ0], bQ1 = B.qc[e + iQ0 + 4];
+            accJ[0] = PipeMfma<T>::step(aJ, B.qv[e + iQV0], accJ[0]);
+            accJ[1] = PipeMfma<T>::step(aJ, B.qv[e + iQV0 + 4], accJ[1]);
+            accJ[2] = PipeMfma<T>::step(aJ, B.qv[e + iQV0 + 32], accJ[2]);
+            accJ[3] = PipeMfma<T>::step(aJ, B.qv[e + iQV0 + 36], accJ[3]);
             accK[0] = PipeMfma<T>::step(aK0, bQ0, accK[0]);
             accK[1] = PipeMfma<T>::step(aK0, bQ1, accK[1]);
             accK[2] = PipeMfma<T>::step(aK1, bQ0, accK[2]);
             accK[3] = PipeMfma<T>::step(aK1, bQ1, accK[3]);
         }
-        if (ch == nch - 1) {
+        if (last) {
 #pragma unroll
             for (int blk = 0; blk < 4; ++blk) {
                 const int chv = blk >> 1, bh = blk & 1;
@@ -994,7 +1022,14 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
                     const T J = sm.xch[w][((kk_of(i) * 4 + cc_of(i)) * 4 + hi) * 4 + lo];
                     const T amat = T(ak) * accK[blk][i] - J;
                     const double am = (double)amat;
-                    double pt = am * am / (dr[chv][i] - dc[bh] + 1.0e-10);
+                    // a reciprocal of two Newton steps: a division's scaling and
+                    // fix-up are half of this epilogue's FP64 instructions
+                    const double den = dr[chv][i] - dc[bh] + 1.0e-10;
+                    double rden = __builtin_amdgcn_rcp(den);
+                    rden = fma(rden, fma(-den, rden, 1.0), rden);
+                    rden = fma(rden, fma(-den, rden, 1.0), rden);
+                    if (den == 0.0) rden = __builtin_inf();
+                    const double pt = am * am * rden;
                     const bool ok = !__builtin_isnan(pt);
                     if (ok) part[chv * 4 + i] += pt;
                     if (ptm)
@@ -1009,8 +1044,11 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
             dc[0] = dcn[0];
             dc[1] = dcn[1];
         }
-        if (more) store(cur ^ 1);
+        cur ^= 1;
+        if (more) store(cur);
         __syncthreads();
+        ch = last ? 0 : ch + 1;
+        other += last ? 1 : 0;
     }
 
 #pragma unroll
