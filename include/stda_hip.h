@@ -317,10 +317,10 @@ int stda_hip_format_curve(int64_t n, const double *e, const double *r, char *out
  *     FP32 with FP32 accumulation, Davidson orthogonalisation, Rayleigh-Ritz
  *     and residual norms in FP64, converged to a residual of 1e-6, followed
  *     by FP64 refinement of the converged roots (TDA: up to four iterations,
- *     to 1e-7; RPA: one Rayleigh-Ritz step).  The response solver uses the
+ *     to 2e-7; RPA: one Rayleigh-Ritz step).  The response solver uses the
  *     FP32 operator with a 1e-6 tolerance.  Molecules too small for the
  *     products' precision to matter in time (below 4e8 flops per vector,
- *     4 nao no (nv + nao)) keep FP64 products, to the same 1e-7.
+ *     4 nao no (nv + nao)) keep FP64 products, to the same 2e-7.
  *   2 split-bfloat16: the same, with the operator GEMMs' FP32 operands split
  *     into two bfloat16 numbers each and multiplied as hi*hi + hi*lo + lo*hi
  *     on the bfloat16 matrix cores with FP32 accumulation, to a residual of

@@ -382,7 +382,6 @@ struct stda_hip_ctx {
     double ak = 2.0, ax = 0.0, thr = 0.0, thrp = 1e-4, fthr = 0.0;
     bool small_ax = false;
     bool have_moments = false;
-    std::vector<double> moments_h;   // 9 * npk (host copy, for window-mode helpers)
     int64_t npk = 0;
 
     // device-resident intermediates
@@ -1366,11 +1365,10 @@ void davidson_rpa(stda_hip_ctx *c, int k, double tol, std::vector<double> &omega
         L.resize((size_t)m * m);
         t1.resize((size_t)m * m);
         Hm.resize((size_t)m * m);
-        for (int j = 0; j < m; ++j)
-            for (int i = 0; i < m; ++i) {
-                ap[i + (size_t)m * j] = 0.5 * (Ap[i + (size_t)maxdim * j] + Ap[j + (size_t)maxdim * i]);
-                L[i + (size_t)m * j] = 0.5 * (Am[i + (size_t)maxdim * j] + Am[j + (size_t)maxdim * i]);
-            }
+        for (int j = 0; j < m; ++j) {   // symmetric as they are stored
+            std::copy_n(Ap.begin() + (size_t)maxdim * j, m, ap.begin() + (size_t)m * j);
+            std::copy_n(Am.begin() + (size_t)maxdim * j, m, L.begin() + (size_t)m * j);
+        }
         if (!host_potrf_lower(m, L))
             throw Error(STDA_HIP_ERR_AMB_NOT_PD, "matrix power impossible (A-B not positive definite)");
         host_gemm(false, false, m, m, m, 1.0, ap.data(), m, L.data(), m, 0.0, t1.data(), m);
@@ -1586,10 +1584,7 @@ static void do_load(stda_hip_ctx *c, const stda_hip_system *sys, const stda_hip_
     c->eps.upload(sys->epsi, moci, s);
     c->have_moments = sys->moments != nullptr;
     c->npk = (int64_t)moci * (moci + 1) / 2;
-    if (c->have_moments) {
-        c->moments.upload(sys->moments, (size_t)9 * c->npk, s);
-        c->moments_h.assign(sys->moments, sys->moments + (size_t)9 * c->npk);
-    }
+    if (c->have_moments) c->moments.upload(sys->moments, (size_t)9 * c->npk, s);
     c->sync();
     c->loaded = true;
 }
@@ -2110,11 +2105,11 @@ static bool fp32_operator(const stda_hip_ctx *c) {
     const double per = 4.0 * c->nao * (double)c->no * (c->nv + (double)c->nao);
     return c->precision == 2 || (c->precision == 1 && per >= 4.0e8);
 }
-constexpr double kMixedTol = 1.0e-7;   // residual tolerance of a mixed-precision solve's FP64 end
+constexpr double kMixedTol = 2.0e-7;   // residual tolerance of a mixed-precision solve's FP64 end
 
 // Mixed precision TDA: FP32 operator to a residual of max(tol, 1e-6), then up to
 // four FP64 iterations: Rayleigh-Ritz in the span of the converged vectors, and
-// three with preconditioned residuals added, or to max(tol, 1e-7).  (The first
+// three with preconditioned residuals added, or to max(tol, 2e-7).  (The first
 // alone leaves the FP32 phase's residual in the vectors, whose rounding makes
 // oscillator strengths scatter by 1e-5 of their size, by up to half from one
 // summation order to another; after two more the error of five 133-atom
@@ -2570,8 +2565,11 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
         }
         std::vector<double> coef;   // (m x 2 nrhs): X+Y coefficients a | X-Y coefficients b
         bool done = mnew == 0;      // no dipole moments at all: alpha = 0
-        std::vector<double> Ap((size_t)maxdim * maxdim), Am((size_t)maxdim * maxdim),
-            Br((size_t)maxdim * 3);
+        // reduced matrices (symmetric, leading dimension maxdim), not initialised:
+        // clearing the 46 MB of each at 2400 vectors took longer than a small solve
+        std::unique_ptr<double[]> Ap(new double[(size_t)maxdim * maxdim]),
+            Am(new double[(size_t)maxdim * maxdim]);
+        std::vector<double> Br((size_t)maxdim * 3);
         std::vector<double> wcol(nrhs);
         for (int f = 0; f < nfreq; ++f)
             for (int r = 0; r < 3; ++r) wcol[f * 3 + r] = omega[f];
@@ -2675,11 +2673,10 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
             // serves the restarts and a breakdown.
             ap.resize((size_t)m * m);
             L.resize((size_t)m * m);
-            for (int j = 0; j < m; ++j)
-                for (int i = 0; i < m; ++i) {
-                    ap[i + (size_t)m * j] = 0.5 * (Ap[i + (size_t)maxdim * j] + Ap[j + (size_t)maxdim * i]);
-                    L[i + (size_t)m * j] = 0.5 * (Am[i + (size_t)maxdim * j] + Am[j + (size_t)maxdim * i]);
-                }
+            for (int j = 0; j < m; ++j) {
+                std::copy_n(Ap.get() + (size_t)maxdim * j, m, ap.begin() + (size_t)m * j);
+                std::copy_n(Am.get() + (size_t)maxdim * j, m, L.begin() + (size_t)m * j);
+            }
             if (!host_potrf_lower(m, L)) throw Error(STDA_HIP_ERR_AMB_NOT_PD, "A-B not positive definite");
             coef.assign((size_t)m * 2 * nrhs, 0.0);
             spectral = false;
@@ -2772,8 +2769,9 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                 c->sync();
                 for (int j = 0; j < m; ++j)
                     for (int i = 0; i < m; ++i) {
-                        Ap[i + (size_t)maxdim * j] = hf[i + (size_t)m * j];
-                        Am[i + (size_t)maxdim * j] = hf[(size_t)m * m + i + (size_t)m * j];
+                        const size_t a = i + (size_t)m * j, b = j + (size_t)m * i, mm = (size_t)m * m;
+                        Ap[i + (size_t)maxdim * j] = 0.5 * (hf[a] + hf[b]);
+                        Am[i + (size_t)maxdim * j] = 0.5 * (hf[mm + a] + hf[mm + b]);
                     }
                 mnew = 0;
                 continue;
@@ -2838,15 +2836,16 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                     STDA_HIP_CHECK(hipMemcpyAsync(B->get(), rs.get(), (size_t)n * r * 8,
                                                   hipMemcpyDeviceToDevice, s));
                 }
-                auto reduce = [&](std::vector<double> &out) {
+                auto reduce = [&](double *out) {
                     std::vector<double> aq((size_t)m * r), qaq((size_t)r * r);
-                    host_gemm(false, false, m, r, m, 1.0, out.data(), maxdim, Q.data(), m, 0.0, aq.data(), m);
+                    host_gemm(false, false, m, r, m, 1.0, out, maxdim, Q.data(), m, 0.0, aq.data(), m);
                     host_gemm(true, false, r, r, m, 1.0, Q.data(), m, aq.data(), m, 0.0, qaq.data(), r);
                     for (int j = 0; j < r; ++j)
-                        for (int i = 0; i < r; ++i) out[i + (size_t)maxdim * j] = qaq[i + (size_t)r * j];
+                        for (int i = 0; i < r; ++i)
+                            out[i + (size_t)maxdim * j] = 0.5 * (qaq[i + (size_t)r * j] + qaq[j + (size_t)r * i]);
                 };
-                reduce(Ap);
-                reduce(Am);
+                reduce(Ap.get());
+                reduce(Am.get());
                 std::vector<double> br((size_t)maxdim * 3, 0.0);
                 host_gemm(true, false, r, 3, m, 1.0, Q.data(), m, Br.data(), maxdim, 0.0, br.data(), maxdim);
                 Br.swap(br);

@@ -85,6 +85,73 @@ def test_root_counts(h, k):
     assert np.abs(sol.X.T @ sol.X - np.eye(k)).max() <= 1e-11
 
 
+def dense_rpa(apb, amb, n):
+    """All RPA roots from the packed A+B and A-B: L^T (A+B) L with A-B = L L^T."""
+    full = []
+    for p in (apb, amb):
+        M = np.zeros((n, n))
+        M[np.tril_indices(n)] = p          # element lin(i, j), j <= i
+        full.append(M + np.tril(M, -1).T)
+    L = np.linalg.cholesky(full[1])
+    return np.sqrt(np.linalg.eigvalsh(L.T @ full[0] @ L)), full
+
+
+@pytest.mark.parametrize("k", [1, 10, 21, 22, 32, 33])
+def test_rpa_root_counts(h, k):
+    """RPA roots with reduced problems on the device (21 roots with their restart pairs) and on
+    the host, blocks orthonormalised on the device (32) and by the host's path (33)."""
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    if not hasattr(test_rpa_root_counts, "ref"):
+        mol, ints = cluster(20, seed=12, basis="minimal")
+        ci = prepare(mol, 7.0, 0.25, ints)
+        h.setup(ci, 7.0, 0.25)
+        test_rpa_root_counts.ref = ci, dense_rpa(*h.build_apb_amb(), h.nci)[0]
+    ci, w = test_rpa_root_counts.ref
+    h.setup(ci, 7.0, 0.25)
+    sol = h.solve_rpa(k)
+    assert np.abs(sol.omega - w[:k]).max() <= 1e-10
+    xpy, xmy = sol.X + sol.Y, sol.X - sol.Y
+    assert np.abs(np.einsum("ij,ij->j", xpy, xmy) - 1.0).max() <= 1e-10
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3, 4])
+@pytest.mark.parametrize("rpa", [False, True])
+def test_window_finds_every_root(h, seed, rpa):
+    """Every root up to the threshold, also where more of them lie there than the CSF
+    energies promise, against the dense eigenvalues."""
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    mol, ints = cluster(14, seed=seed, basis="minimal")
+    ci = prepare(mol, 8.0, 0.5, ints)
+    h.setup(ci, 8.0, 0.5)
+    w = dense_rpa(*h.build_apb_amb(), h.nci)[0] if rpa else np.linalg.eigvalsh(h.build_a())
+    w = w[w <= h.thr]
+    sol = h.solve_rpa(None) if rpa else h.solve_tda(None)
+    assert len(sol.omega) == len(w)
+    assert np.abs(sol.omega - w).max() <= 1e-10
+
+
+@pytest.mark.parametrize("omegas", [(0.0,), (0.0, 0.05, 0.1), (0.05, 0.05, 0.05 + 1e-9), (0.0, 0.3)])
+def test_response_reduced_problem(h, omegas):
+    """alpha(w) below and above poles, and with dependent residuals (equal frequencies: the
+    new block's dead columns leave the space), against a dense solve."""
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    mol, ints = cluster(14, seed=3, basis="minimal")
+    ci = prepare(mol, 7.0, 0.25, ints)
+    h.setup(ci, 7.0, 0.25)
+    P, M = dense_rpa(*h.build_apb_amb(), h.nci)[1]
+    csf = h.csf()[0].astype(int) - 1
+    hi, lo = csf.max(axis=1), csf.min(axis=1)
+    mu = ci.moments[:3, lo + hi * (hi + 1) // 2].T
+    inv = np.linalg.inv(M)
+    for w, a in h.lresp(omegas):
+        ref = 4.0 * mu.T @ np.linalg.solve(P - w * w * inv, mu)
+        # residuals of 1e-10 of norm-1 right-hand sides, amplified by 1 / |w_n - w| at a pole
+        assert np.abs(a - ref).max() <= 1e-6 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("mode,unit", [("fp64", EPS), ("fp32", 2.0 ** -24)])
 @pytest.mark.parametrize("m,n,kk", [(33, 31, 50), (320, 330, 37), (1030, 1050, 37), (2950, 2890, 19)])
 def test_gemm_tile_sizes(h, mode, unit, m, n, kk):
