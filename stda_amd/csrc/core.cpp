@@ -1084,6 +1084,11 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
     bool restarted = false;       // the first m columns are Ritz vectors, H = diag(theta)
     int m = 0, mnew = nguess;
     bool flags_pending = false;   // alive flags of the new block still on the device
+    // no column lives at all: the start vectors (an earlier phase's, from
+    // non-finite data) were not finite
+    auto no_space = [&]() {
+        throw Error(STDA_HIP_ERR_NOT_CONVERGED, "Davidson did not converge (no finite vectors)");
+    };
     if (o.V0) {
         int nv0 = std::min(o.nv0, maxdim);
         STDA_HIP_CHECK(hipMemcpyAsync(V.get(), o.V0, (size_t)n * nv0 * 8, hipMemcpyDeviceToDevice, s));
@@ -1094,6 +1099,7 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
             flags_pending = true;
         } else {
             mnew = orthonormalize(c, V.get(), 0, V.get(), nv0, tmp);
+            if (mnew == 0) no_space();
             std::fill(alive.begin(), alive.begin() + mnew, 1);
         }
     } else {
@@ -1137,6 +1143,7 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
             for (int i = 0; i < mt; ++i)
                 if (alive[i]) idx.push_back(i);
             na = (int)idx.size();
+            if (na == 0) no_space();
             Hs.assign((size_t)na * na, 0.0);
             for (int b = 0; b < na; ++b)
                 for (int a2 = 0; a2 < na; ++a2)
@@ -1178,6 +1185,7 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
             ritz(nrm + k);
             const double *info = rn + 2 * k;
             na = (int)info[1];
+            if (na == 0) no_space();
             const bool stuck = flags_pending && (int)info[2] == 0 && it > 0;
             if (info[0] == 0.0) {   // eigenvalues too close for the kernel: the host's solver
                 std::vector<int> al(mt);

@@ -123,6 +123,13 @@ __global__ void __launch_bounds__(16 * RT, 1) rr_lowest_kernel(RRArgs p) {
     }
     __syncthreads();
     const int na = sm.na, kk = min(p.k, na);
+    if (na == 0) {   // no live column (a start block of non-finite vectors): no pairs, ok = 0
+        const int kc = min(p.k, m);
+        for (int e = tid; e < m * kc; e += T) p.Y[e] = 0.0;
+        if (tid < kc) p.theta[tid] = 0.0;
+        if (tid < 4) p.info[tid] = 0.0;
+        return;
+    }
 
     // the symmetric matrix, kept in H for the next call.  Every element is read
     // by unconditional loads from a chosen address, so that they all overlap.

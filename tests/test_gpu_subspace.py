@@ -165,3 +165,33 @@ def test_gemm_tile_sizes(h, mode, unit, m, n, kk):
             C = h.gemm(A.T if ta else A, B.T if tb else B, ta=ta, tb=tb, mode=mode)
             bound = (kk + 2) * unit * (np.abs(A) @ np.abs(B))
             assert (np.abs(C - A @ B) <= bound + kk * EPS).all()
+
+
+@pytest.mark.parametrize("k", [20, 40, 70])
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "bf16"])
+def test_nonfinite_orbital_is_an_error(h, precision, k):
+    """A NaN in an orbital of no selected CSF (0 times it enters every product) ends in an
+    error, also where a phase starts from the vectors of an earlier one and no column of its
+    start block lives, and the context goes on to the next molecule."""
+    from stda_amd.core import StdaHipError
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    mol, ints = cluster(24, seed=11, basis="minimal")
+    ci = prepare(mol, 7.0, 0.25, ints)
+    good = ci.clow.copy()
+    print(f"non-finite orbital, {precision}, {k} roots", flush=True)
+    try:
+        ci.clow[0, -1] = np.nan
+        h.setup(ci, 7.0, 0.25)
+        h.set_precision(precision)
+        # one phase finds no new directions, a second one no start vectors
+        with pytest.raises(StdaHipError, match="no finite vectors" if precision == "bf16"
+                           else "no new directions") as e:
+            h.solve_tda(k)
+        assert e.value.status == 6       # STDA_HIP_ERR_NOT_CONVERGED
+        ci.clow[:] = good
+        h.setup(ci, 7.0, 0.25)
+        assert np.isfinite(h.solve_tda(k).omega).all()
+    finally:
+        ci.clow[:] = good
+        h.set_precision("fp64")
