@@ -51,6 +51,20 @@ def test_lowest_pairs(h, kind, n):
         assert np.linalg.norm(A @ Z - Z * w, axis=0).max() <= 8 * n * EPS * norm + 1e-14
 
 
+@pytest.mark.parametrize("n", [3, 20, 70, 130, 192])
+def test_scaled_matrices(h, n):
+    """A matrix times a power of two, down to where its elements' squares underflow: the same
+    vectors and the scaled values, bit for bit."""
+    A = matrix("dense", n, np.random.default_rng(n))
+    k = min(n, 20)
+    w, Z = h.sym_lowest(A, k)
+    for e in (-1000, -700, -540, -100, 100, 540, 1000):
+        out = h.sym_lowest(np.ldexp(A, e), k)
+        assert out is not None
+        np.testing.assert_array_equal(out[0], np.ldexp(w, e))
+        np.testing.assert_array_equal(out[1], Z)
+
+
 @pytest.mark.parametrize("n", [4, 40, 100])
 def test_repeated_and_nonfinite(h, n):
     """Repeated eigenvalues and NaN: pairs that hold, or None, and always an end."""
