@@ -1039,6 +1039,11 @@ struct DavOpts {
     double window = 0.0;
 };
 
+// A smaller residual tolerance than asked for, for solves whose roots would come
+// out less exact at tol: not below 1e-11 of its own accord (windows of RPA roots
+// stop at 1e-13 and below, where rounding leaves no new directions).
+double tighter(double tol, double f) { return std::min(tol, std::max(f * tol, 1.0e-11)); }
+
 void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta,
                   DBuf<double> &X, const DavOpts &o = DavOpts()) {
     const int64_t n = c->nci;
@@ -1054,7 +1059,7 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
     // Rayleigh-Ritz on the device (subspace.hip) when the subspace fits its
     // kernel; larger ones on the host
     const bool devrr = k <= RR_KMAX && maxdim <= RR_MMAX;
-    if (small_k) tol *= 0.3;   // another path to the same tolerance: no root less exact
+    if (small_k) tol = tighter(tol, 0.3);   // another path to the same tolerance: no root less exact
     // new blocks of up to 64 directions are orthonormalised on the device
     // (dependent ones stay as zero columns, marked dead; the host learns which
     // with the next Gram block or Ritz values, in the same synchronisation)
@@ -2371,7 +2376,7 @@ int stda_hip_solve_tda(stda_hip_ctx *c, int32_t nroots, int32_t capacity, int32_
             all.window = c->thr;
             // (once enlarged, the roots at the window's edge are no longer those that
             // converge first by far: a smaller tolerance makes up for it)
-            for (double t = tol;; t = 0.02 * tol) {
+            for (double t = tol;; t = tighter(tol, 0.02)) {
                 davidson_tda(c, k, t, w, X, all);
                 if (w.back() > c->thr || k >= n) break;
                 k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));
@@ -2459,7 +2464,7 @@ int stda_hip_solve_rpa(stda_hip_ctx *c, int32_t nroots, int32_t capacity, double
             all.window = c->thr;
             // (once enlarged, the roots at the window's edge are no longer those that
             // converge first by far: a smaller tolerance makes up for it)
-            for (double t = tol;; t = 0.02 * tol) {
+            for (double t = tol;; t = tighter(tol, 0.02)) {
                 davidson_rpa(c, k, t, w, XpY, XmY, all);
                 if (w.back() > c->thr || k >= n) break;
                 k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));

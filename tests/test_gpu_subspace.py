@@ -146,6 +146,28 @@ def test_window_finds_every_root(h, seed, rpa):
     assert np.abs(sol.omega - w).max() <= 1e-10
 
 
+@pytest.mark.parametrize("na,seed,thr,ax,tol,k", [(20, 3, 8.0, 1.0, 1e-12, 0), (24, 4, 6.0, 0.5, 1e-12, 0),
+                                                  (24, 11, 7.0, 0.25, 2e-15, 10),
+                                                  (24, 11, 7.0, 0.25, 2e-15, 19)])
+def test_tolerance_near_rounding(h, na, seed, thr, ax, tol, k):
+    """Tolerances that the iteration just reaches: windows of RPA roots that start too small
+    (k = 0) and fewer than 20 TDA roots, which ask for more than the caller's tolerance."""
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    mol, ints = cluster(na, seed=seed, basis="minimal")
+    h.setup(prepare(mol, thr, ax, ints), thr, ax)
+    if k:
+        w = np.linalg.eigvalsh(h.build_a())[:k]
+        sol = h.solve_tda(k, tol=tol)
+    else:
+        w = dense_rpa(*h.build_apb_amb(), h.nci)[0]
+        w = w[w <= h.thr]
+        assert len(w) > (h.csf()[1] <= h.thr).sum() + 8
+        sol = h.solve_rpa(None, tol=tol)
+    assert len(sol.omega) == len(w)
+    assert np.abs(sol.omega - w).max() <= 1e-10
+
+
 @pytest.mark.parametrize("omegas", [(0.0,), (0.0, 0.05, 0.1), (0.05, 0.05, 0.05 + 1e-9), (0.0, 0.3)])
 def test_response_reduced_problem(h, omegas):
     """alpha(w) below and above poles, and with dependent residuals (equal frequencies: the
