@@ -1033,10 +1033,15 @@ struct DavOpts {
     int nv0 = 0;
     int maxiter = 300;
     bool allow_unconverged = false;
-    // Every root up to this value is wanted (0: the k roots asked for): the solver
-    // returns as soon as k Ritz values lie within it.  They bound the roots from
-    // above, so k roots are too few and iterating them further is in vain.
+    // Every root up to this value is wanted (0: the k roots asked for), and `guard`
+    // of the k are to lie beyond it: the solver returns as soon as more than
+    // k - guard Ritz values lie within.  They bound the roots from above, so k
+    // roots are too few and iterating them further is in vain.
     double window = 0.0;
+    int guard = 1;
+    bool too_few(int k, const std::vector<double> &w) const {
+        return window > 0.0 && w[k - guard] <= window;
+    }
 };
 
 // A smaller residual tolerance than asked for, for solves whose roots would come
@@ -1229,7 +1234,7 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
         }
         m = mt;
         const double *th = devrr ? nrm + k : yt.get() + (size_t)m * kk;
-        if (o.window > 0.0 && kk == k && k < n && theta[k - 1] <= o.window) return;
+        if (kk == k && k < n && o.too_few(k, theta)) return;
         std::vector<int> un;
         for (int j = 0; j < kk; ++j)
             if (!(rn[j] < tol)) un.push_back(j);
@@ -1452,7 +1457,7 @@ void davidson_rpa(stda_hip_ctx *c, int k, double tol, std::vector<double> &omega
         double *rn = pin + o_rn;
         STDA_HIP_CHECK(hipMemcpyAsync(rn, nrm.get(), (size_t)2 * kk * 8, hipMemcpyDeviceToHost, s));
         c->sync();
-        if (o.window > 0.0 && kk == k && k < n && omega[k - 1] <= o.window) return;
+        if (kk == k && k < n && o.too_few(k, omega)) return;
         int nun = 0;
         for (int j = 0; j < 2 * kk; ++j) nun += !(rn[j] < tol);
         if (nun == 0 && kk == k) return;
@@ -2120,6 +2125,34 @@ static bool fp32_operator(const stda_hip_ctx *c) {
 }
 constexpr double kMixedTol = 2.0e-7;   // residual tolerance of a mixed-precision solve's FP64 end
 
+// Every root up to Ethr: solve(k, tol, opts) for the k lowest, from the number of
+// CSF energies in the window plus 8 on, until roots beyond the window show that
+// it holds no more.  A first solve is enlarged when it has none; an enlarged one
+// has to show 8 (the margin that the first one is laid out with): a root that
+// the block missed, or roots at the edge that change places, then cost a value
+// beyond the window and not one inside.  Once enlarged, the roots at the edge are
+// also no longer those that converge first by far: a smaller tolerance makes up
+// for it.
+template <typename F>
+static void window_roots(stda_hip_ctx *c, double tol, std::vector<double> &w, F &&solve) {
+    constexpr int kMargin = 8;
+    const int64_t n = c->nci;
+    int64_t cnt = 0;
+    for (double e : c->ed_h) cnt += e <= c->thr;
+    int k = (int)std::min<int64_t>(n, cnt + kMargin);
+    DavOpts o;
+    o.window = c->thr;
+    for (double t = tol;; t = tighter(tol, 0.02)) {
+        {
+            HostSpan hs(c, "window_solve");
+            solve(k, t, o);
+        }
+        if (k >= n || w[k - o.guard] > c->thr) return;
+        k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));
+        o.guard = kMargin;
+    }
+}
+
 // Mixed precision TDA: FP32 operator to a residual of max(tol, 1e-6), then up to
 // four FP64 iterations: Rayleigh-Ritz in the span of the converged vectors, and
 // three with preconditioned residuals added, or to max(tol, 2e-7).  (The first
@@ -2369,18 +2402,9 @@ int stda_hip_solve_tda(stda_hip_ctx *c, int32_t nroots, int32_t capacity, int32_
             davidson_tda(c, nroots, tol, w, X);
         } else {
             // every root in (0, Ethr] (ssyevr RANGE='V', stda.f:1143-1150)
-            int64_t cnt = 0;
-            for (double e : c->ed_h) cnt += e <= c->thr;
-            int k = (int)std::min<int64_t>(n, cnt + 8);
-            DavOpts all;
-            all.window = c->thr;
-            // (once enlarged, the roots at the window's edge are no longer those that
-            // converge first by far: a smaller tolerance makes up for it)
-            for (double t = tol;; t = tighter(tol, 0.02)) {
-                davidson_tda(c, k, t, w, X, all);
-                if (w.back() > c->thr || k >= n) break;
-                k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));
-            }
+            window_roots(c, tol, w, [&](int k, double t, const DavOpts &o) {
+                davidson_tda(c, k, t, w, X, o);
+            });
             int keep = 0;
             for (double e : w) keep += (e > 0.0 && e <= c->thr);
             int first = 0;
@@ -2457,18 +2481,9 @@ int stda_hip_solve_rpa(stda_hip_ctx *c, int32_t nroots, int32_t capacity, double
         } else if (nroots > 0) {
             davidson_rpa(c, nroots, tol, w, XpY, XmY);
         } else {
-            int64_t cnt = 0;
-            for (double e : c->ed_h) cnt += e <= c->thr;
-            int k = (int)std::min<int64_t>(n, cnt + 8);
-            DavOpts all;
-            all.window = c->thr;
-            // (once enlarged, the roots at the window's edge are no longer those that
-            // converge first by far: a smaller tolerance makes up for it)
-            for (double t = tol;; t = tighter(tol, 0.02)) {
-                davidson_rpa(c, k, t, w, XpY, XmY, all);
-                if (w.back() > c->thr || k >= n) break;
-                k = (int)std::min<int64_t>(n, k + (int64_t)std::max(16, k / 4));
-            }
+            window_roots(c, tol, w, [&](int k, double t, const DavOpts &o) {
+                davidson_rpa(c, k, t, w, XpY, XmY, o);
+            });
             int keep = 0;
             for (double e : w) keep += (e * e <= c->thr * c->thr);   // srpapack.f:84-89
             w.resize(keep);

@@ -146,6 +146,40 @@ def test_window_finds_every_root(h, seed, rpa):
     assert np.abs(sol.omega - w).max() <= 1e-10
 
 
+@pytest.mark.parametrize("edge", [None, 0, 4])
+@pytest.mark.parametrize("na,seed,thr,ax,triplet,rpa", [(24, 5, 4.0, 2.0, True, False),
+                                                        (24, 5, 5.0, 2.0, False, False),
+                                                        (24, 2, 6.0, 1.5, False, False),
+                                                        (20, 3, 8.0, 1.0, False, True),
+                                                        (24, 4, 6.0, 0.5, False, True)])
+def test_window_enlarged(h, na, seed, thr, ax, triplet, rpa, edge):
+    """Windows that hold up to 40 roots more than CSF energies: solved again until 8 roots
+    lie beyond, also for a threshold 1e-6 eV below a root (the highest one, the fifth one)."""
+    from stda_amd.constants import HARTREE_EV
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    mol, ints = cluster(na, seed=seed, basis="minimal")
+
+    def dense(thr):
+        h.setup(prepare(mol, thr, ax, ints), thr, ax, triplet=triplet)
+        return (dense_rpa(*h.build_apb_amb(), h.nci)[0] if rpa else np.linalg.eigvalsh(h.build_a()))
+    w = dense(thr)
+    if edge is not None:
+        thr = w[w <= h.thr][-1 - edge] * HARTREE_EV - 1e-6
+        w = dense(thr)
+    roots = int((w <= h.thr).sum())
+    k, solves = int((h.csf()[1] <= h.thr).sum()) + 8, 1
+    while w[k - (1 if solves == 1 else 8)] <= h.thr:
+        k, solves = k + max(16, k // 4), solves + 1
+    assert solves > 1
+    sol = h.solve_rpa(None) if rpa else h.solve_tda(None)
+    w = w[:roots]
+    w = w[w > 0.0]
+    assert len(sol.omega) == len(w)
+    assert np.abs(sol.omega - w).max() <= 1e-10
+    assert h.kernel_stats("window_solve")["launches"] == solves
+
+
 @pytest.mark.parametrize("na,seed,thr,ax,tol,k", [(20, 3, 8.0, 1.0, 1e-12, 0), (24, 4, 6.0, 0.5, 1e-12, 0),
                                                   (24, 11, 7.0, 0.25, 2e-15, 10),
                                                   (24, 11, 7.0, 0.25, 2e-15, 19)])
