@@ -2629,11 +2629,19 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
         };
         std::vector<double> ap, L, inv, t1, W, Yz, lam;
         bool spectral = false;      // W, Yz and lam are those of the current space
+        // first frequency with the same square, and those whose reduced matrix
+        // was not positive definite when it was last factored
+        std::vector<int> same_as(nfreq);
+        std::vector<char> indef(nfreq, 0);
+        for (int f = 0; f < nfreq; ++f)
+            for (same_as[f] = 0; same_as[f] < f; ++same_as[f])
+                if (std::fabs(omega[same_as[f]]) == std::fabs(omega[f])) break;
         // The space's RPA pairs: with Am = L L^T and L^T Ap L = Z diag(lam) Z^T
         // (lam: the space's w_n^2), W = L Z, Yz = L^-T Z; then a = W c and
         // b = w Yz c with c = (lam - w^2)^-1 W^T V^T r.
         auto spectrum = [&]() {
             if (spectral) return;
+            HostSpan hs(c, "lresp_spectrum");
             std::vector<double> t((size_t)m * m), Z((size_t)m * m);
             host_gemm(false, false, m, m, m, 1.0, ap.data(), m, L.data(), m, 0.0, t.data(), m);
             host_gemm(true, false, m, m, m, 1.0, L.data(), m, t.data(), m, 0.0, Z.data(), m);
@@ -2695,10 +2703,15 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                 m += nk;
             }
             // Reduced problem (Ap - w^2 Am^-1) a = V^T r, b = w Am^-1 a for every
-            // frequency: the inverse of the positive definite Am once, then a
-            // Cholesky (above a pole: symmetric indefinite) solve per frequency.  One eigenproblem for all
-            // of them (below) takes several times as long from 100 vectors on, and
-            // serves the restarts and a breakdown.
+            // frequency.  Few of them: the inverse of the positive definite Am once,
+            // then a Cholesky (above a pole: symmetric indefinite) solve per w^2.
+            // Many: one eigenproblem for all (below), which also serves the
+            // restarts and a breakdown.  For 200 / 400 / 900 vectors it takes 2.87 /
+            // 16.9 / 159 ms, a Cholesky solve 0.126 / 0.67 / 6.2 and an indefinite one
+            // (after the failed Cholesky) 0.20 / 1.06 / 7.6, the inverse 0.27 / 1.6 / 13:
+            // level at 21 / 23 / 24 of the one and 13 / 15 / 19 of the other.  Which
+            // of them are indefinite is taken from the last iteration.  (Below 100
+            // vectors the line lies lower, at 10 for 60, for less than 0.2 ms.)
             ap.resize((size_t)m * m);
             L.resize((size_t)m * m);
             for (int j = 0; j < m; ++j) {
@@ -2708,8 +2721,11 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
             if (!host_potrf_lower(m, L)) throw Error(STDA_HIP_ERR_AMB_NOT_PD, "A-B not positive definite");
             coef.assign((size_t)m * 2 * nrhs, 0.0);
             spectral = false;
-            bool solved = true;
-            if (wmax > 0.0) {
+            double cost = 0.0;
+            for (int f = 0; f < nfreq; ++f)
+                if (same_as[f] == f) cost += !indef[f] ? 1.0 : m < 500 ? 1.6 : 1.3;
+            bool solved = cost <= (m < 300 ? 20.0 : 24.0);
+            if (solved && wmax > 0.0) {
                 inv = L;
                 solved = host_potri(m, inv);
             }
@@ -2721,14 +2737,20 @@ int stda_hip_lresp(stda_hip_ctx *c, int32_t nfreq, const double *omega, double t
                         for (size_t q = 0; q < t1.size(); ++q) t1[q] -= w * w * inv[q];
                 };
                 double *xa = coef.data() + (size_t)m * 3 * f, *xb = coef.data() + (size_t)m * (nrhs + 3 * f);
-                for (int r = 0; r < 3; ++r)
-                    std::copy(Br.begin() + (size_t)maxdim * r, Br.begin() + (size_t)maxdim * r + m,
-                              xa + (size_t)m * r);
-                shifted();   // positive definite below the space's first pole
-                solved = host_potrf_lower(m, t1) && host_potrs(m, 3, t1, xa, m);
-                if (!solved) {
-                    shifted();
-                    solved = host_sysv(m, 3, t1, xa, m);
+                if (same_as[f] < f) {   // the same equations
+                    std::copy_n(coef.begin() + (size_t)m * 3 * same_as[f], (size_t)m * 3, xa);
+                } else {
+                    HostSpan hs(c, "lresp_factor");
+                    for (int r = 0; r < 3; ++r)
+                        std::copy(Br.begin() + (size_t)maxdim * r, Br.begin() + (size_t)maxdim * r + m,
+                                  xa + (size_t)m * r);
+                    shifted();   // positive definite below the space's first pole
+                    solved = host_potrf_lower(m, t1) && host_potrs(m, 3, t1, xa, m);
+                    indef[f] = !solved;
+                    if (!solved) {
+                        shifted();
+                        solved = host_sysv(m, 3, t1, xa, m);
+                    }
                 }
                 if (solved && w != 0.0)
                     host_gemm(false, false, m, 3, m, w, inv.data(), m, xa, m, 0.0, xb, m);

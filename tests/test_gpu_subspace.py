@@ -222,6 +222,40 @@ def test_response_reduced_problem(h, omegas):
         assert np.abs(a - ref).max() <= 1e-6 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("na,seed,below,above,spectral", [(14, 3, 40, 0, True), (24, 11, 20, 20, True),
+                                                          (14, 3, 0, 14, True), (14, 3, 12, 4, False),
+                                                          (14, 3, 20, 0, False)])
+def test_response_many_frequencies(h, na, seed, below, above, spectral):
+    """alpha(w) at many frequencies below the first pole and midway between poles, each but
+    static ones twice with either sign: few are solved one by one (a repeated w^2 once), many
+    through one eigenproblem an iteration."""
+    from stda_amd.prep import prepare
+    from stda_amd.synth import cluster
+    mol, ints = cluster(na, seed=seed, basis="minimal")
+    ci = prepare(mol, 7.0, 0.25, ints)
+    h.setup(ci, 7.0, 0.25)
+    poles, (P, M) = dense_rpa(*h.build_apb_amb(), h.nci)
+    gaps = np.flatnonzero(np.diff(poles) > 2e-3)[:above]
+    w = np.r_[np.linspace(0.0, 0.9, below) * poles[0], 0.5 * (poles[gaps] + poles[gaps + 1])]
+    assert len(w) == below + above
+    w = np.r_[w, -w[::-1]]
+    out = h.lresp(w)
+    factored = h.kernel_stats("lresp_factor")["launches"]
+    if spectral:         # but for iterations before the frequencies are known to lie above poles
+        assert factored <= 2 * (below + above) < 2 * len(w)
+        assert h.kernel_stats("lresp_spectrum")["launches"] > 0
+    else:                # each w^2 once an iteration
+        assert factored > 0 and factored % (below + above) == 0
+    csf = h.csf()[0].astype(int) - 1
+    hi, lo = csf.max(axis=1), csf.min(axis=1)
+    mu = ci.moments[:3, lo + hi * (hi + 1) // 2].T
+    inv = np.linalg.inv(M)
+    for x, a in out:
+        ref = 4.0 * mu.T @ np.linalg.solve(P - x * x * inv, mu)
+        # as in test_response_reduced_problem, half a gap of at least 1e-3 from a pole
+        assert np.abs(a - ref).max() <= 1e-6 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("mode,unit", [("fp64", EPS), ("fp32", 2.0 ** -24)])
 @pytest.mark.parametrize("m,n,kk", [(33, 31, 50), (320, 330, 37), (1030, 1050, 37), (2950, 2890, 19)])
 def test_gemm_tile_sizes(h, mode, unit, m, n, kk):
