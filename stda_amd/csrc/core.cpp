@@ -342,6 +342,18 @@ bool host_sysv(int n, int k, std::vector<double> &a, double *B, int ldb) {
     return info == 0;
 }
 
+// f(); false when the device cannot hold its buffers
+template <typename F>
+bool fits_device(F &&f) {
+    try {
+        f();
+        return true;
+    } catch (const Error &e) {
+        if (e.status != STDA_HIP_ERR_NOMEM) throw;
+        return false;
+    }
+}
+
 struct Timer {
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
     double ms() const {
@@ -3231,8 +3243,6 @@ int stda_hip_ao_ints(stda_hip_ctx *c, int32_t nao, const int64_t *prim_ptr, cons
     })
 }
 
-// Moments and Loewdin orbitals from S and the nine AO matrices, which are host
-// arrays (kind = hipMemcpyHostToDevice) or device buffers (hipMemcpyDeviceToDevice).
 // clow = S^1/2 ca by the coupled Newton-Schulz iteration (Higham, Functions of
 // Matrices, ch. 6): Y_0 = S / s, Z_0 = I, T = (3 I - Z Y) / 2, Y <- Y T, Z <- T Z,
 // Y -> (S / s)^1/2; three products a step, about log_1.5 of the square root of
@@ -3275,35 +3285,59 @@ static bool root_newton_schulz(stda_hip_ctx *c, int64_t na, const double *S, int
     return false;
 }
 
+// moments: shrink(ca^T M_q ca) for the 9 AO matrices (stda.f:351-412,
+// onetri.f:20-55), `group` of them in one launch per product
+static void mo_moments(stda_hip_ctx *c, int64_t na, int64_t nm, const double *ca, const double *ao9,
+                       hipMemcpyKind kind, int group, double *moments) {
+    hipStream_t s = c->stream;
+    const size_t nn = (size_t)na * na;
+    const int64_t npk = nm * (nm + 1) / 2;
+    DBuf<double> T((size_t)group * na * nm), P((size_t)group * nm * nm), A, OUT((size_t)9 * npk);
+    for (int q0 = 0; q0 < 9; q0 += group) {
+        const int g = std::min(group, 9 - q0);
+        const double *m = ao9 + (size_t)q0 * nn;
+        if (kind == hipMemcpyHostToDevice) {
+            A.upload(m, g * nn, s);
+            m = A.get();
+        }
+        dgemm_batched(c->blas, false, false, na, nm, na, 1.0, m, na, na * na, ca, na, 0, 0.0,
+                      T.get(), na, na * nm, g);
+        dgemm_batched(c->blas, true, false, nm, nm, na, 1.0, ca, na, 0, T.get(), na, na * nm, 0.0,
+                      P.get(), nm, nm * nm, g);
+        for (int q = 0; q < g; ++q)
+            launch_pack_upper(s, nm, P.get() + (size_t)q * nm * nm, OUT.get() + (size_t)(q0 + q) * npk);
+    }
+    OUT.download(moments, (size_t)9 * npk, s);
+    c->sync();
+}
+
+// Moments and Loewdin orbitals from S and the nine AO matrices, which are host
+// arrays (kind = hipMemcpyHostToDevice) or device buffers (hipMemcpyDeviceToDevice).
+// The forms that hold more at once (nine matrices a launch, the iteration's four
+// square matrices) give way to those that hold one where the device is too full.
 static void transform_impl(stda_hip_ctx *c, int32_t nao, int32_t moci, const double *ca,
                            const double *S, const double *ao9, hipMemcpyKind kind, int32_t bfw,
                            double *clow, double *moments) {
     hipStream_t s = c->stream;
-    const int64_t na = nao, nm = moci, npk = nm * (nm + 1) / 2;
+    const int64_t na = nao, nm = moci;
     const size_t nn = (size_t)na * na;
-    DBuf<double> CA, M(nn), T((size_t)9 * na * nm), P((size_t)9 * nm * nm), A9;
-    DBuf<double> OUT((size_t)9 * npk);
+    DBuf<double> CA;
     CA.upload(ca, (size_t)na * nm, s);
-    // moments: shrink(ca^T M_q ca) for the 9 AO matrices (stda.f:351-412,
-    // onetri.f:20-55), all nine in one launch per product
-    const double *m9 = ao9;
-    if (kind == hipMemcpyHostToDevice) {
-        A9.upload(ao9, 9 * nn, s);
-        m9 = A9.get();
-    }
-    dgemm_batched(c->blas, false, false, na, nm, na, 1.0, m9, na, na * na, CA.get(), na, 0, 0.0,
-                  T.get(), na, na * nm, 9);
-    dgemm_batched(c->blas, true, false, nm, nm, na, 1.0, CA.get(), na, 0, T.get(), na, na * nm, 0.0,
-                  P.get(), nm, nm * nm, 9);
-    for (int q = 0; q < 9; ++q)
-        launch_pack_upper(s, nm, P.get() + (size_t)q * nm * nm, OUT.get() + (size_t)q * npk);
-    OUT.download(moments, (size_t)9 * npk, s);
+    if (!fits_device([&] { mo_moments(c, na, nm, CA.get(), ao9, kind, 9, moments); }))
+        mo_moments(c, na, nm, CA.get(), ao9, kind, 1, moments);
     // Loewdin: clow = S^1/2 ca (makel, stda.f:1615-1691)
+    DBuf<double> M(nn), CL;
     STDA_HIP_CHECK(hipMemcpyAsync(M.get(), S, nn * 8, kind, s));
-    DBuf<double> CL((size_t)na * nm);
-    if (!root_newton_schulz(c, na, M.get(), nm, CA.get(), CL.get())) {
+    bool have = false;
+    if (!fits_device([&] {
+            CL.resize((size_t)na * nm);
+            have = root_newton_schulz(c, na, M.get(), nm, CA.get(), CL.get());
+        }))
+        device_release_unused();   // the eigensolver's workspace comes from outside the pool
+    if (!have) {
         // through the eigenvalues: U (sqrt(e) o (U^T ca))
-        DBuf<double> D(na), E(na);
+        CL.release();
+        DBuf<double> D(na), E(na), T((size_t)na * nm);
         DBuf<int> info(1);
         STDA_BLAS_CHECK(rocsolver_dsyevd(c->blas, rocblas_evect_original, rocblas_fill_upper,
                                          (rocblas_int)na, M.get(), (rocblas_int)na, D.get(),
@@ -3324,9 +3358,9 @@ static void transform_impl(stda_hip_ctx *c, int32_t nao, int32_t moci, const dou
         D.upload(e.data(), na, s);
         dgemm(c->blas, true, false, na, nm, na, 1.0, M.get(), na, CA.get(), na, 0.0, T.get(), na);
         launch_scale_rows(s, na, nm, D.get(), T.get());
-        dgemm(c->blas, false, false, na, nm, na, 1.0, M.get(), na, T.get(), na, 0.0, CL.get(), na);
+        dgemm(c->blas, false, false, na, nm, na, 1.0, M.get(), na, T.get(), na, 0.0, CA.get(), na);
     }
-    CL.download(clow, (size_t)na * nm, s);
+    (have ? CL : CA).download(clow, (size_t)na * nm, s);
     c->sync();
     // |<c'|c'> - 1| > 1e-2 stops the reference (stda.f:445-450)
     for (int64_t j = 0; j < nm; ++j) {

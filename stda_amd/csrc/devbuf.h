@@ -137,6 +137,20 @@ inline size_t device_available_bytes() {
     return fr > rs ? fr - rs : 0;
 }
 
+// The cached blocks of every stream and the pool's unused memory handed back to
+// the device.
+inline void device_release_unused() {
+    block_cache().drain_all();
+    int dev = 0;
+    hipMemPool_t pool = nullptr;
+    // the released blocks return to the pool in stream order: wait for
+    // them, then hand every unused byte of the pool back
+    if (hipDeviceSynchronize() == hipSuccess && hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
+        (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
+}
+
 inline void *device_alloc(size_t bytes, hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess) cs = hipStreamCaptureStatusNone;
@@ -144,15 +158,7 @@ inline void *device_alloc(size_t bytes, hipStream_t s) {
     const size_t rs = device_reserve_bytes();
     if (cs == hipStreamCaptureStatusNone && hipMemGetInfo(&fr, &tot) == hipSuccess &&
         fr < bytes + rs) {
-        block_cache().drain_all();
-        int dev = 0;
-        hipMemPool_t pool = nullptr;
-        // the released blocks return to the pool in stream order: wait for
-        // them, then hand every unused byte of the pool back
-        if (hipDeviceSynchronize() == hipSuccess && hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
-            (void)hipMemPoolTrimTo(pool, 0);
-        (void)hipGetLastError();
+        device_release_unused();
         if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr < bytes + rs)
             throw Error(STDA_HIP_ERR_NOMEM,
                         "device allocation of " + std::to_string(bytes >> 20) +

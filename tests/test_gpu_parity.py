@@ -238,6 +238,49 @@ def test_device_reserve_nomem():
     assert "status 4" in r.stdout, r.stdout
 
 
+@pytest.mark.parametrize("room_mb", [2000, 420, 195])
+def test_transform_in_little_memory(room_mb):
+    """Moments and Loewdin orbitals of 2000 AOs with 2000 MB beyond the reserve (nine matrices
+    at once take 750), with 420 (one at a time 180, the iteration for S^1/2 210) and with 195
+    (through the eigenvalues): a fresh process each, as the reserve is read once."""
+    import subprocess
+    import textwrap
+    say(f"transforms with {room_mb} MB")
+    code = textwrap.dedent("""
+        import ctypes, os, sys
+        sys.path.insert(0, sys.argv[1])
+        import numpy as np
+        from stda_amd.core import StdaHip
+        rng = np.random.default_rng(1)
+        nao, moci = 2000, 1500
+        X = rng.standard_normal((nao, 40))
+        U, sv, _ = np.linalg.svd(X, full_matrices=False)
+        f = 1.0 + 0.1 * np.arange(40)                   # S = I + U (f - 1) U^T
+        S = np.eye(nao) + (U * (f - 1.0)) @ U.T
+        root = lambda p: np.eye(nao) + (U * (f ** p - 1.0)) @ U.T
+        ca = root(-0.5)[:, :moci]
+        ao9 = [g + g.T for g in rng.standard_normal((9, nao, nao))]
+        with StdaHip(0) as h:
+            hip = ctypes.CDLL("libamdhip64.so")
+            fr, tot = ctypes.c_size_t(), ctypes.c_size_t()
+            assert hip.hipMemGetInfo(ctypes.byref(fr), ctypes.byref(tot)) == 0
+            room = float(sys.argv[2])
+            os.environ["STDA_HIP_DEVICE_RESERVE_MB"] = repr(fr.value / 1048576.0 - room)
+            clow, mom = h.transform(ca, S, ao9)
+        assert np.abs(clow - np.eye(nao)[:, :moci]).max() < 1e-12
+        for q in range(9):
+            M = ca.T @ ao9[q] @ ca
+            packed = M.T[np.tril_indices(moci)]         # lin(i, j) by columns of the triangle
+            assert np.abs(mom[q] - packed).max() < 1e-11 * np.abs(M).max() * np.sqrt(nao)
+        print("ok")
+    """)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code, root, str(room_mb)], env=dict(os.environ),
+                       capture_output=True, text=True, timeout=240, cwd=root)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-2000:]
+    assert "ok" in r.stdout
+
+
 @pytest.mark.parametrize("case", [1, 2, 3])
 def test_water_beta(water, case):
     """SHG beta and beta_HRS (std2 -resp 2) against the reference's BETA_TEST files (its
