@@ -342,7 +342,9 @@ bool host_sysv(int n, int k, std::vector<double> &a, double *B, int ldb) {
     return info == 0;
 }
 
-// f(); false when the device cannot hold its buffers
+// f(); false when the device cannot hold its buffers, which are then given back
+// (a cached block may be up to four times as large as what it is taken for, and
+// rocSOLVER's workspace comes from outside the pool)
 template <typename F>
 bool fits_device(F &&f) {
     try {
@@ -350,8 +352,9 @@ bool fits_device(F &&f) {
         return true;
     } catch (const Error &e) {
         if (e.status != STDA_HIP_ERR_NOMEM) throw;
-        return false;
     }
+    device_release_unused();
+    return false;
 }
 
 struct Timer {
@@ -1056,27 +1059,17 @@ struct DavOpts {
     }
 };
 
-// A smaller residual tolerance than asked for, for solves whose roots would come
-// out less exact at tol: not below 1e-11 of its own accord (windows of RPA roots
-// stop at 1e-13 and below, where rounding leaves no new directions).
-double tighter(double tol, double f) { return std::min(tol, std::max(f * tol, 1.0e-11)); }
-
-void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta,
-                  DBuf<double> &X, const DavOpts &o = DavOpts()) {
+// (in a subspace of up to `space` vectors; davidson_tda below chooses it)
+void davidson_tda_in(stda_hip_ctx *c, int k, int space, double tol, std::vector<double> &theta,
+                     DBuf<double> &X, const DavOpts &o) {
     const int64_t n = c->nci;
     hipStream_t s = c->stream;
-    k = (int)std::min<int64_t>(k, n);
     int nguess = (int)std::min<int64_t>(n, std::max(k + 8, k + k / 2));
-    // Few roots in FP64 get a subspace of 120 as well: 10 roots of a 60-atom
-    // molecule take 30 iterations with 74 vectors and 15 with 120.  (The FP32
-    // phase, whose residuals stop at its own accuracy, keeps its size.)
-    const bool small_k = !o.fp32 && !o.V0 && k < 20;
-    int maxdim = (int)std::min<int64_t>(n, std::max(6 * k, small_k ? 120 : k + 64));
+    int maxdim = (int)std::min<int64_t>(n, space);
     if (maxdim < nguess) maxdim = nguess;
     // Rayleigh-Ritz on the device (subspace.hip) when the subspace fits its
     // kernel; larger ones on the host
     const bool devrr = k <= RR_KMAX && maxdim <= RR_MMAX;
-    if (small_k) tol = tighter(tol, 0.3);   // another path to the same tolerance: no root less exact
     // new blocks of up to 64 directions are orthonormalised on the device
     // (dependent ones stay as zero columns, marked dead; the host learns which
     // with the next Gram block or Ritz values, in the same synchronisation)
@@ -1290,6 +1283,26 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
         }
     }
     throw Error(STDA_HIP_ERR_NOT_CONVERGED, "Davidson did not converge");
+}
+
+// A smaller residual tolerance than asked for, for solves whose roots would come
+// out less exact at tol: not below 1e-11 of its own accord (windows of RPA roots
+// stop at 1e-13 and below, where rounding leaves no new directions).
+double tighter(double tol, double f) { return std::min(tol, std::max(f * tol, 1.0e-11)); }
+
+void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta,
+                  DBuf<double> &X, const DavOpts &o = DavOpts()) {
+    k = (int)std::min<int64_t>(k, c->nci);
+    // Few roots in FP64 get a subspace of 120 as well: 10 roots of a 60-atom
+    // molecule take 30 iterations with 74 vectors and 15 with 120.  (The FP32
+    // phase, whose residuals stop at its own accuracy, keeps its size.)  It is
+    // another path to the same tolerance: 0.3 of it, so that no root is less
+    // exact.  Where the device cannot hold it, the smaller one has to do.
+    if (!o.fp32 && !o.V0 && k < 20 && fits_device([&] {
+            davidson_tda_in(c, k, 120, tighter(tol, 0.3), theta, X, o);
+        }))
+        return;
+    davidson_tda_in(c, k, std::max(6 * k, k + 64), tol, theta, X, o);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -3329,11 +3342,10 @@ static void transform_impl(stda_hip_ctx *c, int32_t nao, int32_t moci, const dou
     DBuf<double> M(nn), CL;
     STDA_HIP_CHECK(hipMemcpyAsync(M.get(), S, nn * 8, kind, s));
     bool have = false;
-    if (!fits_device([&] {
-            CL.resize((size_t)na * nm);
-            have = root_newton_schulz(c, na, M.get(), nm, CA.get(), CL.get());
-        }))
-        device_release_unused();   // the eigensolver's workspace comes from outside the pool
+    (void)fits_device([&] {
+        CL.resize((size_t)na * nm);
+        have = root_newton_schulz(c, na, M.get(), nm, CA.get(), CL.get());
+    });
     if (!have) {
         // through the eigenvalues: U (sqrt(e) o (U^T ca))
         CL.release();

@@ -281,6 +281,40 @@ def test_transform_in_little_memory(room_mb):
     assert "ok" in r.stdout
 
 
+def test_few_roots_in_little_memory():
+    """10 roots of a 100-atom molecule (12 996 CSFs) with 208 MB beyond the reserve: the setup
+    takes 180, a subspace of 74 vectors 24, one of 120 more than the 28 left (a fresh process,
+    as the reserve is read once)."""
+    import subprocess
+    import textwrap
+    say("few roots with little memory")
+    code = textwrap.dedent("""
+        import ctypes, os, sys
+        sys.path.insert(0, sys.argv[1])
+        import numpy as np
+        from stda_amd.core import StdaHip
+        from stda_amd.prep import prepare
+        from stda_amd.synth import cluster
+        mol, ints = cluster(100, seed=3, basis="minimal")
+        ci = prepare(mol, 7.0, 0.25, ints)
+        with StdaHip(0) as h:
+            hip = ctypes.CDLL("libamdhip64.so")
+            fr, tot = ctypes.c_size_t(), ctypes.c_size_t()
+            assert hip.hipMemGetInfo(ctypes.byref(fr), ctypes.byref(tot)) == 0
+            os.environ["STDA_HIP_DEVICE_RESERVE_MB"] = repr(fr.value / 1048576.0 - 208)
+            h.setup(ci, 7.0, 0.25)
+            sol = h.solve_tda(10)
+            res = np.linalg.norm(h.matvec(0, sol.X) - sol.X * sol.omega, axis=0)
+        assert res.max() < 2e-8, res
+        print("ok")
+    """)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code, root], env=dict(os.environ),
+                       capture_output=True, text=True, timeout=240, cwd=root)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-2000:]
+    assert "ok" in r.stdout
+
+
 @pytest.mark.parametrize("case", [1, 2, 3])
 def test_water_beta(water, case):
     """SHG beta and beta_HRS (std2 -resp 2) against the reference's BETA_TEST files (its
