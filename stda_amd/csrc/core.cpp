@@ -423,6 +423,15 @@ struct stda_hip_ctx {
     int precision = 0;    // 0 FP64, 1 FP32 operator + FP64 Davidson numerics and refinement,
                           // 2 split-bfloat16 operator, then FP32, then the FP64 refinement
     int gemm32 = GEMM_F32;   // arithmetic of the FP32 operator's GEMMs in the current phase
+    // A batch's worker: its solves share the device with the other workers' and the
+    // lock step, and are chosen by device time.  Subspace problems go to the host's
+    // LAPACK (sixteen workers have a core each, while their one-work-group kernels of
+    // 0.1 to 0.2 ms stand in four hardware queues before each other's launches),
+    // operator products are FP32 at every size, and one FP64 Rayleigh-Ritz step
+    // follows, as in the lock step.  512 molecules take 780 ms so, 821 with four
+    // FP64 iterations, 854-864 with the other two choices of a context alone, 883
+    // with all three of them.
+    bool worker = false;
     DBuf<float> ct32, gamj32, gamk32;
     DBuf<float> xfull32, tbuf32, dbuf32, gbuf32, wbuf32, rbuf32, ubuf32;
     int nb_max32 = 0;
@@ -1068,8 +1077,8 @@ void davidson_tda_in(stda_hip_ctx *c, int k, int space, double tol, std::vector<
     int maxdim = (int)std::min<int64_t>(n, space);
     if (maxdim < nguess) maxdim = nguess;
     // Rayleigh-Ritz on the device (subspace.hip) when the subspace fits its
-    // kernel; larger ones on the host
-    const bool devrr = k <= RR_KMAX && maxdim <= RR_MMAX;
+    // kernel; larger ones, and those of a batch's worker, on the host
+    const bool devrr = !c->worker && k <= RR_KMAX && maxdim <= RR_MMAX;
     // new blocks of up to 64 directions are orthonormalised on the device
     // (dependent ones stay as zero columns, marked dead; the host learns which
     // with the next Gram block or Ritz values, in the same synchronisation)
@@ -2140,13 +2149,14 @@ static void tda_properties(stda_hip_ctx *c, const double *X, const std::vector<d
 }
 
 // Whether a mixed-precision solve uses the FP32 operator: from 4e8 flops per vector
-// and product on (about 165 atoms in a minimal basis).  Below, an iteration is
+// and product on (about 165 atoms in a minimal basis), a batch's worker always.
+// Below, an iteration is
 // launches and the subspace step, the product's precision hardly shows in its
 // time (133 atoms, 20 vectors: 0.19 ms in FP64, 0.12 in FP32, of 0.6), and FP64
 // throughout to the refinement's tolerance needs three iterations fewer.
 static bool fp32_operator(const stda_hip_ctx *c) {
     const double per = 4.0 * c->nao * (double)c->no * (c->nv + (double)c->nao);
-    return c->precision == 2 || (c->precision == 1 && per >= 4.0e8);
+    return c->precision == 2 || (c->precision == 1 && (c->worker || per >= 4.0e8));
 }
 constexpr double kMixedTol = 2.0e-7;   // residual tolerance of a mixed-precision solve's FP64 end
 
@@ -2184,7 +2194,8 @@ static void window_roots(stda_hip_ctx *c, double tol, std::vector<double> &w, F 
 // alone leaves the FP32 phase's residual in the vectors, whose rounding makes
 // oscillator strengths scatter by 1e-5 of their size, by up to half from one
 // summation order to another; after two more the error of five 133-atom
-// molecules was 0.35 to 1.0 times that, for 6 % of a solve.)  With the
+// molecules was 0.35 to 1.0 times that, for 6 % of a solve.  A batch's worker keeps
+// to the first, as the lock step does.)  With the
 // split-bfloat16 operator (precision 2) a first phase runs to 3e-5 (about its
 // noise floor) and the FP32 phase starts from its Ritz vectors.
 static void solve_tda_mixed(stda_hip_ctx *c, int nroots, double tol, std::vector<double> &w,
@@ -2211,7 +2222,7 @@ static void solve_tda_mixed(stda_hip_ctx *c, int nroots, double tol, std::vector
     DavOpts ref;
     ref.V0 = X.get();
     ref.nv0 = (int)w.size();
-    ref.maxiter = 4;
+    ref.maxiter = c->worker ? 1 : 4;
     ref.allow_unconverged = true;
     DBuf<double> X0 = std::move(X);
     HostSpan hs(c, "mixed_fp64_refine");
@@ -4358,6 +4369,7 @@ int stda_hip_batch_create(stda_hip_batch **out, int device, int nworkers) {
             return st;
         }
         c->precision = 1;
+        c->worker = true;
         b->workers.push_back(c);
     }
     b->device = b->workers[0]->device;

@@ -79,6 +79,30 @@ def test_batch_matches_fp64(molecules, plain):
         np.testing.assert_allclose(pr[:, :2], rpr[:, :2], atol=F_MIX, rtol=0)
 
 
+def test_batch_worker_solves(molecules):
+    """A worker's own solves are laid out for the shared device: FP32 products at every size,
+    subspace problems on the host, one FP64 step at the end (and the velocity correction's
+    product), while a context alone solves the same molecules in FP64 with the kernel."""
+    from stda_amd.core import StdaHip, StdaHipBatch
+    stats = lambda x: {k: x.kernel_stats(k)["launches"] for k in
+                       ("ao_matvec", "ao_matvec_f32", "dav_rr_eig", "mixed_fp64_refine")}
+    with StdaHipBatch(0, workers=2) as b:
+        b.configure(nmax_batched=4096)
+        b.configure_wide(False)
+        res = b.solve_tda(molecules[-2:], 7.0, 0.25, nroots=20)
+        assert b.timings()[1]["single"] == 2
+        k = stats(b)
+    assert all(st == 0 for _, _, st in res)
+    assert k["ao_matvec"] == 4 and k["mixed_fp64_refine"] == 2
+    assert k["ao_matvec_f32"] == k["dav_rr_eig"] - 2 > 2
+    with StdaHip(0) as h:
+        h.setup(molecules[-1], 7.0, 0.25)
+        h.set_precision("mixed")
+        h.solve_tda(20)
+        k = stats(h)
+    assert k["ao_matvec"] > 2 and k["ao_matvec_f32"] == k["dav_rr_eig"] == k["mixed_fp64_refine"] == 0
+
+
 def test_batch_bf16_single_path(molecules, plain):
     """Split-bfloat16 operator products on the single-molecule path of the
     workers (stda_hip_batch_set_precision 2): same bar against plain FP64."""
