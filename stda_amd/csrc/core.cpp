@@ -2150,13 +2150,20 @@ static void tda_properties(stda_hip_ctx *c, const double *X, const std::vector<d
 
 // Whether a mixed-precision solve uses the FP32 operator: from 4e8 flops per vector
 // and product on (about 165 atoms in a minimal basis), a batch's worker always.
-// Below, an iteration is
-// launches and the subspace step, the product's precision hardly shows in its
-// time (133 atoms, 20 vectors: 0.19 ms in FP64, 0.12 in FP32, of 0.6), and FP64
-// throughout to the refinement's tolerance needs three iterations fewer.
+// Below, FP64 products to the refinement's tolerance are as fast for a context
+// alone: of launches and subspace steps there are three iterations fewer.  FP32
+// phase and refinement against FP64 throughout, ms for 5, 10 and 20 TDA roots:
+// 5.2, 9.9, 11.1 against 5.2, 8.7, 11.2 at 2.1e8 (133 atoms), 5.8, 8.7, 10.9
+// against 5.8, 7.8, 11.0 at 2.7e8, 6.5, 7.6, 11.5 against 6.6, 7.1, 11.7 at 4.0e8,
+// 8.0, 10.7, 15.1 against 8.7, 10.0, 15.9 at 7.0e8 (200 atoms).  Response: 9.9
+// against 8.0 at 2.1e8.  RPA pays for the exactness (24 against 28 ms for 10 roots
+// at 2.1e8, 26 against 36 at 1.2e8): its FP32 form ends with one FP64 step from
+// residuals of 1e-6.  STDA_HIP_FP32_MIN_FLOPS sets another line (for tests).
 static bool fp32_operator(const stda_hip_ctx *c) {
-    const double per = 4.0 * c->nao * (double)c->no * (c->nv + (double)c->nao);
-    return c->precision == 2 || (c->precision == 1 && (c->worker || per >= 4.0e8));
+    if (c->precision != 1 || c->worker) return c->precision >= 1;
+    double line = 4.0e8;
+    if (const char *e = getenv("STDA_HIP_FP32_MIN_FLOPS")) line = std::strtod(e, nullptr);
+    return 4.0 * c->nao * (double)c->no * (c->nv + (double)c->nao) >= line;
 }
 constexpr double kMixedTol = 2.0e-7;   // residual tolerance of a mixed-precision solve's FP64 end
 

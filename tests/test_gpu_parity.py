@@ -713,3 +713,37 @@ def test_mixed_precision_tda_rpa(polyene, cluster30):
     refa = O.run(polyene, 7.0, 0.25, rpa=True, resp_omegas=[0.0, 0.05])
     for (w, a), (wr, ar) in zip(res, refa.alpha_resp):
         np.testing.assert_allclose(a, ar, rtol=0, atol=1e-4 * np.abs(ar).max())
+
+
+@pytest.mark.parametrize("line", ["0", "1e30"])
+def test_mixed_precision_either_operator(polyene, cluster30, monkeypatch, line):
+    """The same with the FP32 operator and with FP64 products, whatever the molecule's size."""
+    monkeypatch.setenv("STDA_HIP_FP32_MIN_FLOPS", line)
+    with _hip() as h:
+        h.setup(polyene, 7.0, 0.25)
+        h.set_precision("mixed")
+        for solve in (lambda: h.solve_tda(8), lambda: h.solve_rpa(8), lambda: h.lresp([0.05])):
+            before = h.kernel_stats("ao_matvec_f32")["launches"]
+            solve()
+            assert (h.kernel_stats("ao_matvec_f32")["launches"] > before) == (line == "0")
+    test_mixed_precision_tda_rpa(polyene, cluster30)
+
+
+@pytest.mark.parametrize("seed,fp32", [(1, True), (2, False)])
+def test_mixed_precision_at_the_line(seed, fp32):
+    """165 atoms on either side of the 4e8 flops per vector from which a mixed-precision solve
+    takes the FP32 operator (4.02e8, 3.91e8), against the plain FP64 solve."""
+    from stda_amd import synth
+    mol, ints = synth.cluster(165, seed=seed, basis="minimal")
+    ci = prepare(mol, 7.0, 0.25, ints)
+    flops = 4.0 * ci.nao * ci.no * (ci.nv + ci.nao)
+    say(f"mixed precision, 165 atoms, {flops:.3g} flops per vector")
+    assert (flops >= 4e8) == fp32 and abs(flops / 4e8 - 1.0) < 0.05
+    with _hip() as h:
+        h.setup(ci, 7.0, 0.25)
+        ref = h.solve_tda(20)
+        h.set_precision("mixed")
+        sol = h.solve_tda(20)
+        assert (h.kernel_stats("ao_matvec_f32")["launches"] > 0) == fp32
+    assert np.abs(sol.omega - ref.omega).max() < MIXED_E_TOL
+    np.testing.assert_allclose(sol.props[:, :2], ref.props[:, :2], atol=MIXED_F_TOL, rtol=0)
