@@ -1022,14 +1022,7 @@ __global__ void __launch_bounds__(256, 2) pt2_pipe_kernel(
                     const T J = sm.xch[w][((kk_of(i) * 4 + cc_of(i)) * 4 + hi) * 4 + lo];
                     const T amat = T(ak) * accK[blk][i] - J;
                     const double am = (double)amat;
-                    // a reciprocal of two Newton steps: a division's scaling and
-                    // fix-up are half of this epilogue's FP64 instructions
-                    const double den = dr[chv][i] - dc[bh] + 1.0e-10;
-                    double rden = __builtin_amdgcn_rcp(den);
-                    rden = fma(rden, fma(-den, rden, 1.0), rden);
-                    rden = fma(rden, fma(-den, rden, 1.0), rden);
-                    if (den == 0.0) rden = __builtin_inf();
-                    const double pt = am * am * rden;
+                    const double pt = am * am / (dr[chv][i] - dc[bh] + 1.0e-10);
                     const bool ok = !__builtin_isnan(pt);
                     if (ok) part[chv * 4 + i] += pt;
                     if (ptm)
