@@ -299,3 +299,17 @@ def test_nonfinite_orbital_is_an_error(h, precision, k):
     finally:
         ci.clow[:] = good
         h.set_precision("fp64")
+
+
+@pytest.mark.parametrize("mode,unit", [("fp64", EPS), ("fp32", 2.0 ** -24)])
+def test_gemm_tuned_small_tiles(h, mode, unit):
+    """A product large enough to be tuned (2.1 GFLOP) whose 64-tiles are fewer than the compute
+    units: the tuning call and the calls after it, which use the tile it chose."""
+    rng = np.random.default_rng(5)
+    m, n, kk = 650, 610, 2700
+    A, B = rng.standard_normal((m, kk)), rng.standard_normal((kk, n))
+    if mode == "fp32":
+        A, B = A.astype(np.float32).astype(float), B.astype(np.float32).astype(float)
+    bound = (kk + 2) * unit * (np.abs(A) @ np.abs(B)) + kk * EPS
+    for _ in range(3):
+        assert (np.abs(h.gemm(A, B, mode=mode) - A @ B) <= bound).all()
