@@ -73,10 +73,12 @@ def _selection_sort_quirk(eps, C_full, moci):
     """sort_vec: selection sort of eps(1:moci), swapping columns of C_full."""
     eps = eps.copy()
     swapped = False
-    if (np.diff(eps[:moci]) >= 0.0).all():
+    if (eps[1:moci] >= eps[:moci - 1]).all():
         return eps, False        # ascending: no strictly smaller value anywhere
     for i in range(moci - 1):
-        k = i + int(np.argmin(eps[i:moci]))      # the first minimum
+        if np.isnan(eps[i]):     # nothing compares smaller
+            continue
+        k = i + int(np.nanargmin(eps[i:moci]))   # the first minimum
         if eps[k] < eps[i]:
             eps[[i, k]] = eps[[k, i]]
             C_full[:, [i, k]] = C_full[:, [k, i]]

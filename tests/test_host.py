@@ -3,6 +3,7 @@ boundary preparation, and the serving scheduler's bookkeeping."""
 import os
 
 import numpy as np
+import pytest
 
 from stda_amd import synth
 from stda_amd.molden import read_molden, write_molden
@@ -116,3 +117,36 @@ def test_primary_order_is_the_reference_selection_sort(tmp_path):
             assert out.tolist() == ref
             differs += ref != np.argsort(keys, kind="stable").tolist()
     assert differs > 0
+
+
+@pytest.mark.parametrize("kind", ["ascending", "random", "ties", "nan", "inf"])
+def test_selection_sort_of_energies(kind):
+    """sort_vec's order and column swaps, element by element as the reference's loops run:
+    repeated energies, NaN (which compares smaller than nothing) and infinities included."""
+    from stda_amd.prep import _selection_sort_quirk
+    rng = np.random.default_rng(3)
+    for n in (0, 1, 2, 7, 40):
+        e = rng.uniform(-1.0, 1.0, n + 3)
+        if kind == "ascending":
+            e.sort()
+        elif kind == "ties":
+            e = np.round(e, 1)
+        elif kind == "nan":
+            e[rng.permutation(n + 3)[:1 + n // 5]] = np.nan
+        elif kind == "inf":
+            e[rng.permutation(n + 3)[:2]] = np.inf, -np.inf
+        ref, cols, moved = e.copy(), np.arange(n + 3.0)[None].copy(), False
+        for i in range(n - 1):
+            k = i
+            for j in range(i + 1, n):
+                if ref[j] < ref[k]:
+                    k = j
+            if k != i:
+                ref[[i, k]] = ref[[k, i]]
+                cols[:, [i, k]] = cols[:, [k, i]]
+                moved = True
+        C = np.arange(n + 3.0)[None].copy()
+        got, swapped = _selection_sort_quirk(e, C, n)
+        np.testing.assert_array_equal(got, ref)
+        np.testing.assert_array_equal(C, cols)
+        assert swapped == moved
