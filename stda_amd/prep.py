@@ -73,7 +73,7 @@ def _selection_sort_quirk(eps, C_full, moci):
     """sort_vec: selection sort of eps(1:moci), swapping columns of C_full."""
     eps = eps.copy()
     swapped = False
-    if (eps[1:moci] >= eps[:moci - 1]).all():
+    if moci < 2 or (eps[1:moci] >= eps[:moci - 1]).all():
         return eps, False        # ascending: no strictly smaller value anywhere
     for i in range(moci - 1):
         if np.isnan(eps[i]):     # nothing compares smaller
