@@ -3788,7 +3788,15 @@ int stda_hip_sym_lowest(stda_hip_ctx *c, int32_t n, int32_t k, const double *a, 
         const size_t nn = (size_t)n * n;
         DBuf<double> G, H(nn + (size_t)RR_MMAX * RR_MMAX), Y((size_t)n * k), rep((size_t)k + 4);
         DBuf<int> live(n);
-        G.upload(a, nn, s);
+        // The largest element scaled to about one: the kernel sums squares as they
+        // are.  A power of two changes no rounding.
+        double big = 0.0;
+        for (size_t q = 0; q < nn; ++q) big = std::max(big, std::fabs(a[q]));
+        int ex = 0;
+        if (std::isfinite(big)) (void)std::frexp(big, &ex);
+        std::vector<double> as(nn);
+        for (size_t q = 0; q < nn; ++q) as[q] = std::ldexp(a[q], -ex);
+        G.upload(as.data(), nn, s);
         RRArgs ra{};
         ra.mnew = n;
         ra.k = k;
@@ -3805,7 +3813,7 @@ int stda_hip_sym_lowest(stda_hip_ctx *c, int32_t n, int32_t k, const double *a, 
         rep.download(r.data(), r.size(), s);
         Y.download(z, (size_t)n * k, s);
         c->sync();
-        std::copy(r.begin(), r.begin() + k, w);
+        for (int j = 0; j < k; ++j) w[j] = std::ldexp(r[j], ex);
         *ok = r[k] != 0.0 ? 1 : 0;
     })
 }

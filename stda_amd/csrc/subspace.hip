@@ -28,6 +28,9 @@
 //
 // The matrix H itself stays on the device: the kernel adds the new columns'
 // Gram block (mirrored) and keeps the result for the next iteration.
+//
+// Squares of the elements are summed unscaled: the largest element is to lie well
+// within 1e-150 .. 1e150 (the solvers' are energies; stda_hip_sym_lowest scales).
 
 #include "common.h"
 
@@ -135,7 +138,6 @@ __global__ void __launch_bounds__(16 * RT, 1) rr_lowest_kernel(RRArgs p) {
     // by unconditional loads from a chosen address, so that they all overlap.
     // Lanes of a grid row read neighbouring rows of a column of H or gram.
     double A[NR][NC];
-    int sexp;   // A holds the matrix times 2^-sexp
     {
         int ir[NR], ic[NC];
 #pragma unroll
@@ -161,27 +163,13 @@ __global__ void __launch_bounds__(16 * RT, 1) rr_lowest_kernel(RRArgs p) {
                 A[a][b] = in && !zero ? 0.5 * (u[b] + v[b]) : 0.0;
             }
         }
-        double big = 0.0;
-#pragma unroll
-        for (int a = 0; a < NR; ++a)
-#pragma unroll
-            for (int b = 0; b < NC; ++b) big = fmax(big, fabs(A[a][b]));
-        for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
-        if (lane == 0) sm.red[wave] = big;
         __syncthreads();   // every element of H (and theta) read before any is written
 #pragma unroll
-        for (int q = 0; q < T / 64; ++q) big = fmax(big, sm.red[q]);
-        // the largest element scaled into [1/2, 1): the squares below neither
-        // underflow nor overflow, and a power of two changes no rounding
-        sexp = big > 0.0 && big < __builtin_inf() ? __builtin_amdgcn_frexp_exp(big) : 0;
-#pragma unroll
         for (int a = 0; a < NR; ++a)
 #pragma unroll
-            for (int b = 0; b < NC; ++b) {
+            for (int b = 0; b < NC; ++b)
                 if (tr + RT * a < na && tc + 16 * b < na)
                     p.H[ic[b] + (int64_t)p.ldh * ir[a]] = A[a][b];
-                A[a][b] = __builtin_amdgcn_ldexp(A[a][b], -sexp);
-            }
     }
 
     // 1. tridiagonalisation; the owners of column j write it, diagonal included.
@@ -561,7 +549,7 @@ __global__ void __launch_bounds__(16 * RT, 1) rr_lowest_kernel(RRArgs p) {
             const int i = tc + 16 * a, c = tr + RT * q;
             if (i < na && c < kk) p.Y[sm.idx[i] + (int64_t)m * c] = y[q][a];
         }
-    if (tid < kc) p.theta[tid] = tid < kk ? __builtin_amdgcn_ldexp(sm.lam[tid] * tn, sexp) : 0.0;
+    if (tid < kc) p.theta[tid] = tid < kk ? sm.lam[tid] * tn : 0.0;
     if (tid == 0) {
         p.info[0] = sm.bad ? 0.0 : 1.0;
         p.info[1] = (double)na;
