@@ -318,9 +318,11 @@ int stda_hip_format_curve(int64_t n, const double *e, const double *r, char *out
  *     and residual norms in FP64, converged to a residual of 1e-6, followed
  *     by FP64 refinement of the converged roots (TDA: up to four iterations,
  *     to 2e-7; RPA: one Rayleigh-Ritz step).  The response solver uses the
- *     FP32 operator with a 1e-6 tolerance.  Molecules too small for the
- *     products' precision to matter in time (below 4e8 flops per vector,
- *     4 nao no (nv + nao)) keep FP64 products, to the same 2e-7.
+ *     FP32 operator with a 1e-6 tolerance, then FP64.  Molecules too small for
+ *     the products' precision to matter in time (below 4e8 flops per vector,
+ *     4 nao no (nv + nao); STDA_HIP_FP32_MIN_FLOPS sets another line) keep FP64
+ *     products, to the same 2e-7.  A batch's solves, whose workers share the
+ *     device, use FP32 products at every size and one FP64 step.
  *   2 split-bfloat16: the same, with the operator GEMMs' FP32 operands split
  *     into two bfloat16 numbers each and multiplied as hi*hi + hi*lo + lo*hi
  *     on the bfloat16 matrix cores with FP32 accumulation, to a residual of
@@ -342,8 +344,10 @@ int stda_hip_gemm(stda_hip_ctx *ctx, int32_t mode, int32_t ta, int32_t tb, int32
 
 /* The k lowest eigenpairs of a symmetric matrix (n x n, column-major; n <= 192,
  * k <= min(n, 32)) with the kernel of the eigensolver's subspace step: w[k]
- * ascending, z (n x k) orthonormal.  *ok = 0 when eigenvalues lie too close for
- * it (then w and z are not to be used; the solvers take the host's LAPACK).
+ * ascending, z (n x k) orthonormal.  The matrix is scaled by a power of two
+ * first, so that its magnitude does not matter.  *ok = 0 when eigenvalues lie too
+ * close for it or an element is not finite (then w and z are not to be used; the
+ * solvers take the host's LAPACK).
  * No counterpart in the reference (its ssyevr/ssyevd); exposes the kernel to
  * tests and to callers that want it. */
 int stda_hip_sym_lowest(stda_hip_ctx *ctx, int32_t n, int32_t k, const double *a, double *w,

@@ -541,7 +541,7 @@ struct stda_hip_ctx {
             STDA_HIP_CHECK(hipStreamSynchronize(stream));
             if (pin) (void)hipHostFree(pin);
             pin = nullptr;
-            n = std::max(n, 2 * pin_n);   // growing spaces ask for a little more each time
+            n = std::max(n, 2 * pin_n);   // doubled: growing spaces ask for more each time
             pin_n = 0;
             STDA_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), n * sizeof(double), 0));
             pin_n = n;
@@ -1316,8 +1316,8 @@ void davidson_tda(stda_hip_ctx *c, int k, double tol, std::vector<double> &theta
 
 // ------------------------------------------------------------------------------------------
 // Paired Davidson for the RPA problem (A-B)(A+B)|X+Y> = w^2 |X+Y>, using
-// the Hermitian reduced form (Am^1/2 Ap Am^1/2) of the subspace problem so
-// that (A-B)^1/2 is never formed in the full space.
+// the Hermitian reduced form L^T Ap L of the subspace problem, Am = L L^T, so
+// that no root of A-B is formed in the full space.
 void davidson_rpa(stda_hip_ctx *c, int k, double tol, std::vector<double> &omega,
                   DBuf<double> &XpY, DBuf<double> &XmY, const DavOpts &o = DavOpts()) {
     const int64_t n = c->nci;
@@ -3277,7 +3277,8 @@ int stda_hip_ao_ints(stda_hip_ctx *c, int32_t nao, const int64_t *prim_ptr, cons
 // clow = S^1/2 ca by the coupled Newton-Schulz iteration (Higham, Functions of
 // Matrices, ch. 6): Y_0 = S / s, Z_0 = I, T = (3 I - Z Y) / 2, Y <- Y T, Z <- T Z,
 // Y -> (S / s)^1/2; three products a step, about log_1.5 of the square root of
-// the condition number steps (24 for 500 AOs in a split-valence basis).  The
+// the condition number steps (12 for 768 AOs in a minimal basis, 15 for 500 in a
+// split-valence one; condition numbers 51 and 780).  The
 // eigensolve below it replaces as the usual way took 17 of 20 ms on the device
 // for 768 AOs, in 3600 launches of a few microseconds each.  False when it does
 // not converge, as for an indefinite or singular S.

@@ -768,9 +768,10 @@ namespace stda {
 // (tile, atom chunk) steps are flattened; while the matrix cores work on step
 // s from one LDS buffer, the operands of step s+1 are fetched into registers
 // and then written to the other buffer, so a single barrier per step orders
-// everything.  The matrix cores bound it (59 % busy at 180 atoms in a split-valence
-// basis before the addresses were kept and the LDS conflicts went, 41 TFLOP/s of
-// couplings; 115 -> 102 ms there, 5.28 -> 4.79 ms at 200 atoms in a minimal basis).
+// everything.  The matrix cores bound it: 59 % busy at 180 atoms in a split-valence
+// basis (41 TFLOP/s of couplings) before the addresses were kept and the LDS
+// conflicts went, which took 115 ms to 102 there and 5.28 to 4.8-4.9 at 200 atoms
+// in a minimal basis.
 // LDS rows of 68 elements: in FP64 the two rows that half a wave reads then fall
 // into distinct banks (65 left every read with conflicts, 17 % of the LDS time),
 // and rows 8.. shift by 4 more so that the writes do too.
@@ -1427,6 +1428,20 @@ __global__ void col_norm_final_kernel(int nsl, int k, const double *part, double
     norms[c] = sqrt(s);
 }
 
+// LDS operations of a wave complete in order: keeps the compiler from moving them
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// value of lane `lane` (uniform), in scalar registers
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 // Cholesky factor of the Gram matrix S = T^T T (nt x nt, nt <= 64) of a
 // block of directions, dependent ones dropped, and the transposed inverse of
 // the factor on the kept columns: LinvT (nt x nt, ld nt), so that T LinvT is
@@ -1447,21 +1462,8 @@ __global__ void col_norm_final_kernel(int nsl, int k, const double *part, double
 // |t_j|, and column k of T LinvT carries at most that sum of them: at the
 // bound it stays below about 1e-13 and another projection of T LinvT against
 // V would change nothing that matters, so the caller may leave it out.
-// LDS operations of a wave complete in order: keeps the compiler from moving them
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// value of lane `lane` (uniform), in scalar registers
-__device__ __forceinline__ double lane_value(double x, int lane) {
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_readlane((int)b, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// NT: registers of a row, nt <= NT
+//
+// NT: registers of a row, nt <= NT.
 template <int NT>
 __global__ __launch_bounds__(256) void chol_inv_kernel(int nt, const double *__restrict__ G, int m,
                                                        int ldg, const double *__restrict__ ref,
@@ -1531,8 +1533,10 @@ __global__ __launch_bounds__(256) void chol_inv_kernel(int nt, const double *__r
     // the factor reaches the other lanes as scalars (readlane).  Four waves with
     // the matrix in LDS took two barriers a column: 24 us for the kernel at
     // nt = 20 and m = 100, 31 us for one wave on LDS; 16 us this way, 9 us for
-    // nt <= 16.  The code is straight and read once, so a size has a kernel
-    // with no more of it than it needs.
+    // nt <= 16.  Above 48 columns, launches one after the other at m = 100: 139 to
+    // 228 us (nt = 49, 64) before, 59 to 70 now; among a solve's other kernels 78
+    // to 96.  The code is straight and read once, so a size has a kernel with no
+    // more of it than it needs.
     double row[NT];
 #pragma unroll
     for (int k = 0; k < NT; ++k) row[k] = lane < nt && k < nt ? L[lane * 65 + k] : 0.0;
