@@ -428,8 +428,8 @@ struct stda_hip_ctx {
     // LAPACK (sixteen workers have a core each, while their one-work-group kernels of
     // 0.1 to 0.2 ms stand in four hardware queues before each other's launches),
     // operator products are FP32 at every size, and one FP64 Rayleigh-Ritz step
-    // follows, as in the lock step.  512 molecules take 780 ms so, 821 with four
-    // FP64 iterations, 854-864 with the other two choices of a context alone, 883
+    // follows, as in the lock step.  512 molecules take 765-780 ms so, 821 with four
+    // FP64 iterations, 854 with the other two choices of a context alone, 881-890
     // with all three of them.
     bool worker = false;
     DBuf<float> ct32, gamj32, gamk32;
